@@ -75,8 +75,8 @@ enum sr_error {
 #define SR_LANE_ELEMENTS 4
 #define SR_LANE_ELEMENTS_NARROW 8
 
-/* Row flag: every pointer of the row is 16-byte aligned, so full tiles take
- * the 128-bit vector path.  Rows without it take the coalesced scalar path. */
+/* Row flag: every pointer of the row is 16-byte aligned.  Hosts may set it;
+ * the kernels move rows of any alignment the same way. */
 #define SR_ROW_VECTOR 1u
 /* Row flag: `param_index` already holds the update key (functional API);
  * the kernel then skips the on-device key derivation. */

@@ -138,8 +138,6 @@ int tiles_for(int64_t n, int block, int lanes, uint32_t* tiles) {
   return SR_OK;
 }
 
-bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
-
 sr::AdamWScalars adamw_scalars(const sr_adamw_hparams& h) {
   return {h.beta1, h.beta2, h.one_minus_beta1, h.one_minus_beta2,
           h.neg_step_size, h.correction2_sqrt, h.decay, h.eps, 1.0f / h.correction2_sqrt};
@@ -302,7 +300,6 @@ int sr_cast(const void* x, void* y, int64_t n, int dtype, int rule, uint32_t see
   a.y = y;
   a.n = n;
   a.counter_base = seed + offset;
-  a.vector_ok = aligned16(x) && aligned16(y);
   if (int rc = tiles_for(n, block_size, sr::kCastLaneElements, &a.total_tiles)) return rc;
   const bool cached_loads = n <= sr::kCachedCastMaxElements;
   return launch(tables().cast[cached_loads][enc], block_size, a.total_tiles, &a, stream);
@@ -358,8 +355,7 @@ int sr_adamw_step(void* p, const void* g, void* m, void* v, int64_t n, int p_dty
   r.tile_end = a.total_tiles;
   r.param_index = key;
   r.shard_start = offset;
-  r.flags = SR_ROW_KEYED |
-            ((aligned16(p) && aligned16(g) && aligned16(m) && aligned16(v)) ? SR_ROW_VECTOR : 0u);
+  r.flags = SR_ROW_KEYED;
   return launch(tables().adamw[pi][gi][me][ve], block_size, a.total_tiles, &a, stream,
                 adamw_cap(pi, gi, me, ve, block_size, a.total_tiles));
 }
@@ -420,7 +416,7 @@ int sr_sgdm_step(void* p, const void* g, void* u, int64_t n, int p_dtype, int g_
   r.tile_end = a.total_tiles;
   r.param_index = key;
   r.shard_start = offset;
-  r.flags = SR_ROW_KEYED | ((aligned16(p) && aligned16(g) && aligned16(u)) ? SR_ROW_VECTOR : 0u);
+  r.flags = SR_ROW_KEYED;
   return launch(tables().sgdm[pi][gi][ue], block_size, a.total_tiles, &a, stream,
                 sgdm_cap(pi, gi, ue, block_size, a.total_tiles));
 }

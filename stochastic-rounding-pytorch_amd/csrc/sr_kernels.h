@@ -8,9 +8,13 @@
 // accesses below, E = 4 is the faster optimizer width for every combination
 // tried (E4M3 + BF16 moments 6.03 vs 5.41 TB/s at E = 8, BF16 parameters
 // and momentum 6.47 vs 6.21) and E = 8 the faster cast width (BF16 output
-// 6.08 vs 5.81 TB/s).  Rows whose pointers are not all 16-byte
-// aligned, and the partial last tile of a row, take a coalesced scalar path
-// (element k*blockDim.x + lane of the tile).
+// 6.08 vs 5.81 TB/s).  Rows of any alignment take the same accesses: a
+// group's alignment is declared as one element's (GroupAccess), which gfx950
+// serves with the same instructions.  Measured on MI355X against one access
+// per element for rows off 16-byte alignment, per launch: FP16-SR moments on
+// packed FP32 gradients, 230 M elements 882 -> 700 us, 49 M 177 -> 155;
+// BF16 with E5M2-SR m, 13 M 38.8 -> 32.5.  The partial last tile of a row
+// takes whole groups too, and its last lanes the 1-3 elements after them.
 //
 // XCD-aware order.  Workgroups map to tiles through sr_tile_order.h: each
 // XCD takes chunks of up to 512 consecutive tiles in turn, so the tiles in
@@ -70,7 +74,6 @@ struct CastArgs {
   int64_t n;
   uint32_t counter_base;  // seed + offset (mod 2^32)
   uint32_t total_tiles;
-  uint32_t vector_ok;     // x and y 16-byte aligned
 };
 
 // Logical tile of this workgroup; >= total_tiles for the padding workgroups.
@@ -105,9 +108,6 @@ __device__ __forceinline__ SR_GLOBAL T* gptr_mut(void* p) {
 // per launch, so every global load and store carries the non-temporal hint.
 // Measured on MI355X: north star 5.64 -> 6.13 TB/s, SGDM 5.87 -> 6.41 TB/s;
 // the hint on loads alone is slower (5.51) and on stores alone neutral.
-typedef uint32_t stream_v4 __attribute__((ext_vector_type(4)));
-typedef uint32_t stream_v2 __attribute__((ext_vector_type(2)));
-
 template <class T>
 __device__ __forceinline__ T stream_load(const void* p) {
   return __builtin_nontemporal_load(gptr<T>(p));
@@ -117,51 +117,40 @@ __device__ __forceinline__ void stream_store(void* p, T v) {
   __builtin_nontemporal_store(v, gptr_mut<T>(p));
 }
 
-// E elements at index i (i a multiple of E, base 16-byte aligned), moved as
-// one access of E * width bytes (two for 32 bytes).  kCached keeps a 16-byte
-// load under the normal cache policy (the small casts' input, below).
+// The words of one group of four elements, moved as one access.  The types
+// promise the alignment of one element only, so groups of views that start
+// anywhere move the same way: gfx950's global accesses take any alignment,
+// and an access that is aligned costs what a declared alignment would.
+template <int BYTES>
+struct GroupAccess;
+template <>
+struct GroupAccess<16> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4))); };
+template <>
+struct GroupAccess<8> { typedef uint32_t type __attribute__((ext_vector_type(2), aligned(2))); };
+template <>
+struct GroupAccess<4> { typedef uint32_t type __attribute__((aligned(1))); };
+
+// kCached keeps the load under the normal cache policy (the small casts'
+// input, below).
 template <int BYTES, bool kCached = false>
 __device__ __forceinline__ void load_words(const char* ptr, uint32_t* w) {
-  static_assert(!kCached || BYTES == 16, "cached loads are 16-byte loads");
-  if constexpr (kCached) {
-    const stream_v4 a = *gptr<stream_v4>(ptr);
-    w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w;
-  } else if constexpr (BYTES == 32) {
-    const stream_v4 a = stream_load<stream_v4>(ptr), b = stream_load<stream_v4>(ptr + 16);
-    w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w; w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
-  } else if constexpr (BYTES == 16) {
-    const stream_v4 a = stream_load<stream_v4>(ptr);
-    w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w;
-  } else if constexpr (BYTES == 8) {
-    const stream_v2 a = stream_load<stream_v2>(ptr);
-    w[0] = a.x; w[1] = a.y;
-  } else if constexpr (BYTES == 4) {
-    w[0] = stream_load<uint32_t>(ptr);
-  } else {
-    static_assert(BYTES == 2, "unsupported access width");
-    w[0] = stream_load<uint16_t>(ptr);
-  }
+  using T = typename GroupAccess<BYTES>::type;
+  T a;
+  if constexpr (kCached) a = *gptr<T>(ptr);
+  else a = stream_load<T>(ptr);
+  __builtin_memcpy(w, &a, BYTES);
 }
 
 template <int BYTES>
 __device__ __forceinline__ void store_words(char* ptr, const uint32_t* w) {
-  if constexpr (BYTES == 32) {
-    stream_store(ptr, stream_v4{w[0], w[1], w[2], w[3]});
-    stream_store(ptr + 16, stream_v4{w[4], w[5], w[6], w[7]});
-  } else if constexpr (BYTES == 16) {
-    stream_store(ptr, stream_v4{w[0], w[1], w[2], w[3]});
-  } else if constexpr (BYTES == 8) {
-    stream_store(ptr, stream_v2{w[0], w[1]});
-  } else if constexpr (BYTES == 4) {
-    stream_store(ptr, w[0]);
-  } else {
-    static_assert(BYTES == 2, "unsupported access width");
-    stream_store(ptr, static_cast<uint16_t>(w[0]));
-  }
+  using T = typename GroupAccess<BYTES>::type;
+  T a;
+  __builtin_memcpy(&a, w, BYTES);
+  stream_store<T>(ptr, a);
 }
 
-// The storage words of the group of four elements at index i (a multiple
-// of four, base 16-byte aligned), moved as one access.
+// The storage words of the group of four elements at index i, moved as one
+// access.
 template <int ENC, bool kCached = false>
 __device__ __forceinline__ void load_group(const void* base, int64_t i, uint32_t (&words)[group_words(ENC)]) {
   load_words<kGroup * enc_bytes(ENC), kCached>(static_cast<const char*>(base) + i * enc_bytes(ENC), words);
@@ -226,6 +215,23 @@ __device__ __forceinline__ uint32_t row_key(const Args& a, const sr_row& r) {
   return (r.flags & SR_ROW_KEYED)
              ? r.param_index
              : update_key_from_prefix(a.key_prefix, r.param_index);
+}
+
+// Elements of this workgroup's tile, which starts `left` elements before its
+// row's end.
+template <int E>
+__device__ __forceinline__ uint32_t tile_count(int64_t left) {
+  const int64_t tile = blockDim.x * E;
+  return static_cast<uint32_t>(left < 0 ? 0 : (left < tile ? left : tile));
+}
+
+// The element of the tile that this lane takes beside the groups of E: the
+// last lanes take the count % E elements after the last whole group, the
+// others get an index at or past `count`.  The last wave of a partial tile
+// mostly has no group, so its remainder runs beside the other waves' groups.
+template <int E>
+__device__ __forceinline__ uint32_t remainder_element(uint32_t count) {
+  return (count & ~static_cast<uint32_t>(E - 1)) + (blockDim.x - 1 - threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -326,18 +332,15 @@ __global__ __launch_bounds__(kMaxBlock) void adamw_kernel(const AdamWArgs a) {
   const uint32_t key = row_key(a, r);
   const uint32_t cm = state_key(key, 0) + r.shard_start;
   const uint32_t cv = state_key(key, 1) + r.shard_start;
-  const uint32_t tile = blockDim.x * E;
-  const int64_t start = static_cast<int64_t>(t - r.tile_begin) * tile;
-  if ((r.flags & SR_ROW_VECTOR) && start + tile <= numel) {
+  const int64_t start = static_cast<int64_t>(t - r.tile_begin) * (blockDim.x * E);
+  const uint32_t count = tile_count<E>(numel - start);
+  if (threadIdx.x < count / E) {
     adamw_vector<PE, GE, ME, VE>(p + start * enc_bytes(PE), g + start * enc_bytes(GE), m + start * enc_bytes(ME),
                                  v + start * enc_bytes(VE), threadIdx.x,
                                  static_cast<uint32_t>(start) + threadIdx.x * E, cm, cv, s);
-  } else {
-#pragma unroll
-    for (int k = 0; k < E; ++k) {
-      const int64_t i = start + static_cast<int64_t>(k) * blockDim.x + threadIdx.x;
-      if (i < numel) adamw_scalar<PE, GE, ME, VE>(p, g, m, v, i, cm, cv, s);
-    }
+  }
+  if (const uint32_t e = remainder_element<E>(count); e < count) {
+    adamw_scalar<PE, GE, ME, VE>(p, g, m, v, start + e, cm, cv, s);
   }
 }
 
@@ -387,17 +390,14 @@ __global__ __launch_bounds__(kMaxBlock) void sgdm_kernel(const SgdmArgs a) {
   char* u = reinterpret_cast<char*>(r.ptr[2]);
   const int64_t numel = r.numel;
   const uint32_t cu = state_key(row_key(a, r), 0) + r.shard_start;
-  const uint32_t tile = blockDim.x * E;
-  const int64_t start = static_cast<int64_t>(t - r.tile_begin) * tile;
-  if ((r.flags & SR_ROW_VECTOR) && start + tile <= numel) {
+  const int64_t start = static_cast<int64_t>(t - r.tile_begin) * (blockDim.x * E);
+  const uint32_t count = tile_count<E>(numel - start);
+  if (threadIdx.x < count / E) {
     sgdm_vector<PE, GE, UE>(p + start * enc_bytes(PE), g + start * enc_bytes(GE), u + start * enc_bytes(UE),
                             threadIdx.x, static_cast<uint32_t>(start) + threadIdx.x * E, cu, a.s);
-  } else {
-#pragma unroll
-    for (int k = 0; k < E; ++k) {
-      const int64_t i = start + static_cast<int64_t>(k) * blockDim.x + threadIdx.x;
-      if (i < numel) sgdm_scalar<PE, GE, UE>(p, g, u, i, cu, a.s);
-    }
+  }
+  if (const uint32_t e = remainder_element<E>(count); e < count) {
+    sgdm_scalar<PE, GE, UE>(p, g, u, start + e, cu, a.s);
   }
 }
 
@@ -427,10 +427,10 @@ __global__ __launch_bounds__(kMaxBlock) void cast_kernel(const CastArgs a) {
   constexpr int E = kCastLaneElements, G = kCastGroup;
   const uint32_t t = logical_tile(a.total_tiles);
   if (t >= a.total_tiles) return;
+  static_assert(G == kGroup, "cast groups are encoder groups");
   const uint32_t tile = blockDim.x * E;
   const int64_t start = static_cast<int64_t>(t) * tile;
-  if (a.vector_ok && start + tile <= a.n) {
-    static_assert(G == kGroup, "cast groups are encoder groups");
+  if (start + tile <= a.n) {
     uint32_t r[E / G][G];
 #pragma unroll
     for (int k = 0; k < E / G; ++k) {
@@ -447,13 +447,30 @@ __global__ __launch_bounds__(kMaxBlock) void cast_kernel(const CastArgs a) {
       store_group<ENC>(a.y, i, words);
     }
   } else {
+    // The last tile: the same groups where they fit, all loaded before the
+    // first is encoded, and the last n % 4 elements one by one.
+    const uint32_t count = static_cast<uint32_t>(a.n - start);
+    uint32_t r[E / G][G];
 #pragma unroll
-    for (int k = 0; k < E; ++k) {
-      const int64_t i = start + static_cast<int64_t>(k) * blockDim.x + threadIdx.x;
-      if (i < a.n) {
-        const float x = bits_f32(load1<ENC_F32>(a.x, i));
-        store1<ENC>(a.y, i, encode<ENC>(x, a.counter_base + static_cast<uint32_t>(i)));
+    for (int k = 0; k < E / G; ++k) {
+      const uint32_t j = k * blockDim.x + threadIdx.x;
+      if (j < count / G) load_group<ENC_F32, kCachedLoads>(a.x, start + j * G, r[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < E / G; ++k) {
+      const uint32_t j = k * blockDim.x + threadIdx.x;
+      if (j < count / G) {
+        float x[G];
+#pragma unroll
+        for (int e = 0; e < G; ++e) x[e] = bits_f32(r[k][e]);
+        uint32_t words[group_words(ENC)];
+        encode_group<ENC, true>(x, a.counter_base + static_cast<uint32_t>(start) + j * G, words);
+        store_group<ENC>(a.y, start + j * G, words);
       }
+    }
+    if (const uint32_t e = remainder_element<G>(count); e < count) {
+      const int64_t i = start + e;
+      store1<ENC>(a.y, i, encode<ENC>(bits_f32(load1<ENC_F32>(a.x, i)), a.counter_base + static_cast<uint32_t>(i)));
     }
   }
 }
