@@ -37,9 +37,16 @@
 //
 // set_steps(entries, value)
 //   entry["step"] = value for every dict in the list ``entries``.
+//
+// observed() -> bool
+//   Whether anything in this process or thread would see a profiler range:
+//   a record-function callback (every profiler, of this thread or global)
+//   or a torch dispatch mode.
 
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <ATen/record_function.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <structmember.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -398,6 +405,10 @@ PyObject* set_steps(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
+PyObject* observed(PyObject*, PyObject*) {
+  return PyBool_FromLong(at::hasCallbacks() || c10::impl::TorchDispatchModeTLS::any_modes_set());
+}
+
 // enable_spec_fast_path(spec_type): compare DTensor gradient specs of this
 // exact type with specs_certainly_equal before falling back to __eq__.  The
 // caller vouches that the type's equality is its mesh, placements, shard
@@ -442,6 +453,7 @@ PyMethodDef kMethods[] = {
     {"group_signature", group_signature, METH_VARARGS,
      "group_signature(params, state, state_names, uses_step, first_index)"},
     {"spans_disjoint", spans_disjoint, METH_VARARGS, "spans_disjoint(spans) -> bool"},
+    {"observed", observed, METH_NOARGS, "observed() -> bool"},
     {"set_steps", set_steps, METH_VARARGS, "set_steps(entries, value)"},
     {nullptr, nullptr, 0, nullptr},
 };

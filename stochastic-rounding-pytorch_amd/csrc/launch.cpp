@@ -1,5 +1,5 @@
-// Native entries of the single-tensor launches: the standalone cast and the
-// functional AdamW and momentum-SGD updates.
+// Native entries of the launches: the standalone cast, the functional AdamW
+// and momentum-SGD updates, and the optimizers' multi-tensor launches.
 //
 // A launch over up to a few million elements is bound by the host: the HIP
 // launch itself costs about 2.2 us, and reaching it through a Python wrapper
@@ -9,9 +9,26 @@
 // their messages, and calls the C ABI's entry points through the addresses
 // the Python side binds once.
 //
-// bind(cast, adamw_step, sgdm_step)
-//   Keep the addresses of sr_cast, sr_adamw_step and sr_sgdm_step, taken
-//   from the loaded library.
+// bind(cast, adamw_step, sgdm_step[, adamw_multi, sgdm_multi])
+//   Keep the addresses of sr_cast, sr_adamw_step, sr_sgdm_step,
+//   sr_adamw_multi and sr_sgdm_multi, taken from the loaded library.
+//
+// cast_new(x, dtype_code, rule, seed, offset, threads, stream) -> tensor, int or None
+//   cast() into a new contiguous tensor of x's shape and device, allocated
+//   here as torch.empty_like allocates it: about 1.5 us less per call than
+//   allocating in Python.  Returns the tensor, or the entry's status where
+//   that is not 0.  None, with nothing allocated, for an x that is not
+//   exactly a torch.Tensor or Parameter, or under a __torch_function__ mode:
+//   there the allocation belongs to the subclass or the mode.
+//
+// adamw_multi(rows, tile_rows, row_scalars, nrows, total_tiles, p, g, m,
+//             m_rule, v, v_rule, hparams, seed, rng_step, block_size, device,
+//             stream) -> int
+// sgdm_multi(rows, tile_rows, nrows, total_tiles, p, g, u, u_rule, hparams,
+//            seed, rng_step, block_size, device, stream) -> int
+//   sr_adamw_multi and sr_sgdm_multi with GPU number `device` current; tables
+//   and hparams are addresses (row_scalars 0 for none), borrowed for the call.
+//   Through ctypes the same call costs 3 us more.
 //
 // cast(x, out, dtype_code, rule, seed, offset, threads, stream) -> int
 //   x: contiguous FP32 tensor; out: contiguous tensor of x's shape and
@@ -33,7 +50,7 @@
 //   Python float.  Raises TypeError or ValueError before anything is
 //   launched; nothing is launched for empty tensors.
 //
-// Each entry calls the C ABI with the first tensor's device current (set and
+// Each tensor entry calls the C ABI with the first tensor's device current (set and
 // restored only when it is not) and the GIL released, and returns its
 // status.  Non-empty tensors without device memory (wrapper subclasses) are
 // refused with ValueError.  seed, key and offset are taken modulo 2^32;
@@ -41,6 +58,8 @@
 
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/ops/empty_like.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -58,9 +77,15 @@ using AdamWFn = int (*)(void*, const void*, void*, void*, int64_t, int, int, int
                         const sr_adamw_hparams*, uint32_t, uint32_t, int, void*);
 using SgdmFn = int (*)(void*, const void*, void*, int64_t, int, int, int, int, const sr_sgdm_hparams*, uint32_t,
                        uint32_t, int, void*);
+using AdamWMultiFn = int (*)(const sr_row*, const uint32_t*, const float*, int, uint32_t, int, int, int, int, int, int,
+                             const sr_adamw_hparams*, uint64_t, uint64_t, int, void*);
+using SgdmMultiFn = int (*)(const sr_row*, const uint32_t*, int, uint32_t, int, int, int, int, const sr_sgdm_hparams*,
+                            uint64_t, uint64_t, int, void*);
 CastFn g_cast = nullptr;
 AdamWFn g_adamw = nullptr;
 SgdmFn g_sgdm = nullptr;
+AdamWMultiFn g_adamw_multi = nullptr;
+SgdmMultiFn g_sgdm_multi = nullptr;
 
 // sr_dtype codes of include/sr_states_hip.h.
 bool dtype_matches(int code, c10::ScalarType type) {
@@ -82,12 +107,14 @@ PyObject* fail(PyObject* type, const char* message) {
 void* address(unsigned long long value) { return reinterpret_cast<void*>(static_cast<uintptr_t>(value)); }
 
 PyObject* bind(PyObject*, PyObject* args) {
-  unsigned long long cast = 0, adamw = 0, sgdm = 0;
-  if (!PyArg_ParseTuple(args, "KKK", &cast, &adamw, &sgdm)) return nullptr;
+  unsigned long long cast = 0, adamw = 0, sgdm = 0, adamw_multi = 0, sgdm_multi = 0;
+  if (!PyArg_ParseTuple(args, "KKK|KK", &cast, &adamw, &sgdm, &adamw_multi, &sgdm_multi)) return nullptr;
   if (!cast || !adamw || !sgdm) return fail(PyExc_ValueError, "null entry point address");
   g_cast = reinterpret_cast<CastFn>(address(cast));
   g_adamw = reinterpret_cast<AdamWFn>(address(adamw));
   g_sgdm = reinterpret_cast<SgdmFn>(address(sgdm));
+  g_adamw_multi = reinterpret_cast<AdamWMultiFn>(address(adamw_multi));
+  g_sgdm_multi = reinterpret_cast<SgdmMultiFn>(address(sgdm_multi));
   Py_RETURN_NONE;
 }
 
@@ -100,17 +127,17 @@ bool tensors(std::initializer_list<PyObject*> objects) {
 
 // Calls `launch` with `device` current and the GIL released, as torch's
 // own operators and a ctypes call do (a launch can wait for room in the
-// device queue); a device the guard cannot select becomes a RuntimeError.
-// The tensors stay alive through the caller's argument tuple.
+// device queue).  False, with a RuntimeError set, for a C++ exception, such
+// as a device that the guard cannot select.  The tensors stay alive through
+// the caller's argument tuple.
 template <class Launch>
-PyObject* on_device(const c10::Device& device, Launch launch) {
-  int status = 0;
+bool run_on_device(const c10::Device& device, Launch launch) {
   bool failed = false;
   std::string message;
   Py_BEGIN_ALLOW_THREADS
   try {
     const c10::DeviceGuard guard(device);
-    status = launch();
+    launch();
   } catch (const std::exception& error) {
     failed = true;
     message = error.what();
@@ -119,7 +146,15 @@ PyObject* on_device(const c10::Device& device, Launch launch) {
     message = "unknown C++ exception in a native launch";
   }
   Py_END_ALLOW_THREADS
-  if (failed) return fail(PyExc_RuntimeError, message.c_str());
+  if (failed) fail(PyExc_RuntimeError, message.c_str());
+  return !failed;
+}
+
+// The same for a launch that returns its status.
+template <class Launch>
+PyObject* on_device(const c10::Device& device, Launch launch) {
+  int status = 0;
+  if (!run_on_device(device, [&] { status = launch(); })) return nullptr;
   return PyLong_FromLong(status);
 }
 
@@ -157,6 +192,41 @@ PyObject* cast(PyObject*, PyObject* args) {
     return g_cast(x.const_data_ptr(), out.data_ptr(), n, code, rule, static_cast<uint32_t>(seed),
                   static_cast<uint32_t>(offset), threads, address(stream));
   });
+}
+
+c10::ScalarType scalar_type(int code) {
+  switch (code) {
+    case SR_BF16: return c10::ScalarType::BFloat16;
+    case SR_F16: return c10::ScalarType::Half;
+    case SR_E4M3: return c10::ScalarType::Float8_e4m3fn;
+    case SR_E5M2: return c10::ScalarType::Float8_e5m2;
+    default: return c10::ScalarType::Float;
+  }
+}
+
+PyObject* cast_new(PyObject*, PyObject* args) {
+  PyObject* x_obj;
+  int code, rule, threads;
+  unsigned long long seed, offset, stream;
+  if (!PyArg_ParseTuple(args, "OiiKKiK", &x_obj, &code, &rule, &seed, &offset, &threads, &stream)) return nullptr;
+  if (!THPVariable_CheckExact(x_obj) || at::impl::torch_function_mode_enabled()) Py_RETURN_NONE;
+  const at::Tensor& x = THPVariable_Unpack(x_obj);
+  if (code < SR_F32 || code > SR_E5M2) return fail(PyExc_ValueError, "unknown cast dtype");
+  if (!x.is_cuda() || x.scalar_type() != c10::ScalarType::Float || !x.is_contiguous()) {
+    return fail(PyExc_ValueError, "the cast input must be a contiguous FP32 tensor on the GPU");
+  }
+  if (g_cast == nullptr) return fail(PyExc_RuntimeError, "the native entries are not bound to the library");
+  at::Tensor out;
+  int status = 0;
+  const bool ran = run_on_device(x.device(), [&] {
+    out = at::empty_like(x, x.options().dtype(scalar_type(code)), at::MemoryFormat::Contiguous);
+    if (x.numel() == 0) return;
+    TORCH_CHECK_VALUE(x.const_data_ptr() != nullptr, "tensors without device memory cannot be cast");
+    status = g_cast(x.const_data_ptr(), out.data_ptr(), x.numel(), code, rule, static_cast<uint32_t>(seed),
+                    static_cast<uint32_t>(offset), threads, address(stream));
+  });
+  if (!ran) return nullptr;
+  return status ? PyLong_FromLong(status) : THPVariable_Wrap(std::move(out));
 }
 
 // The tensor checks of the fused updates, in the validating order of
@@ -279,6 +349,39 @@ PyObject* sgdm_step(PyObject*, PyObject* args) {
   });
 }
 
+PyObject* adamw_multi(PyObject*, PyObject* args) {
+  unsigned long long rows, tile_rows, row_scalars, hparams, seed, rng_step, stream;
+  unsigned int total_tiles;
+  int nrows, p, g, m, m_rule, v, v_rule, block, device;
+  if (!PyArg_ParseTuple(args, "KKKiIiiiiiiKKKiiK", &rows, &tile_rows, &row_scalars, &nrows, &total_tiles, &p, &g, &m,
+                        &m_rule, &v, &v_rule, &hparams, &seed, &rng_step, &block, &device, &stream)) {
+    return nullptr;
+  }
+  if (g_adamw_multi == nullptr) return fail(PyExc_RuntimeError, "the native entries are not bound to the library");
+  return on_device(c10::Device(c10::DeviceType::CUDA, static_cast<c10::DeviceIndex>(device)), [&] {
+    return g_adamw_multi(static_cast<const sr_row*>(address(rows)), static_cast<const uint32_t*>(address(tile_rows)),
+                         static_cast<const float*>(address(row_scalars)), nrows, total_tiles, p, g, m, m_rule, v,
+                         v_rule, static_cast<const sr_adamw_hparams*>(address(hparams)), seed, rng_step, block,
+                         address(stream));
+  });
+}
+
+PyObject* sgdm_multi(PyObject*, PyObject* args) {
+  unsigned long long rows, tile_rows, hparams, seed, rng_step, stream;
+  unsigned int total_tiles;
+  int nrows, p, g, u, u_rule, block, device;
+  if (!PyArg_ParseTuple(args, "KKiIiiiiKKKiiK", &rows, &tile_rows, &nrows, &total_tiles, &p, &g, &u, &u_rule,
+                        &hparams, &seed, &rng_step, &block, &device, &stream)) {
+    return nullptr;
+  }
+  if (g_sgdm_multi == nullptr) return fail(PyExc_RuntimeError, "the native entries are not bound to the library");
+  return on_device(c10::Device(c10::DeviceType::CUDA, static_cast<c10::DeviceIndex>(device)), [&] {
+    return g_sgdm_multi(static_cast<const sr_row*>(address(rows)), static_cast<const uint32_t*>(address(tile_rows)),
+                        nrows, total_tiles, p, g, u, u_rule, static_cast<const sr_sgdm_hparams*>(address(hparams)),
+                        seed, rng_step, block, address(stream));
+  });
+}
+
 // Every entry behind one guard: a C++ exception from torch (a tensor
 // without storage refuses its data pointer) becomes a RuntimeError instead
 // of escaping into the interpreter.
@@ -294,7 +397,10 @@ PyObject* guarded(PyObject* self, PyObject* args) {
 }
 
 PyMethodDef methods[] = {
-    {"bind", bind, METH_VARARGS, "Keep the addresses of the C ABI's single-tensor entry points."},
+    {"bind", bind, METH_VARARGS, "Keep the addresses of the C ABI's entry points."},
+    {"cast_new", guarded<cast_new>, METH_VARARGS, "Cast into a new tensor; returns it, a nonzero status, or None."},
+    {"adamw_multi", guarded<adamw_multi>, METH_VARARGS, "Call sr_adamw_multi on a device; returns its status."},
+    {"sgdm_multi", guarded<sgdm_multi>, METH_VARARGS, "Call sr_sgdm_multi on a device; returns its status."},
     {"cast", guarded<cast>, METH_VARARGS, "Check the tensors and call sr_cast; returns its status."},
     {"adamw_step", guarded<adamw_step>, METH_VARARGS,
      "Check the tensors and call sr_adamw_step; returns its status."},
@@ -302,7 +408,7 @@ PyMethodDef methods[] = {
     {nullptr, nullptr, 0, nullptr},
 };
 
-PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", "Native entries of the single-tensor launches.", -1, methods};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", "Native entries of the launches.", -1, methods};
 
 }  // namespace
 

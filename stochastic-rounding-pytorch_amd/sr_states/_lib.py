@@ -195,18 +195,27 @@ def on_device(device: torch.device):
     return torch.cuda.device(device)
 
 
+_is_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", None) or torch.cuda.is_current_stream_capturing
+
+
+def capturing() -> bool:
+    """Whether the current stream is under graph capture (never before torch has initialized the GPU)."""
+    return torch.cuda.is_initialized() and _is_capturing()
+
+
 _launcher = None
 
 
 def launcher():
-    """The native entries of the single-tensor launches (sr_states/_launch), bound to this library."""
+    """The native entries of the launches (sr_states/_launch), bound to this library."""
     global _launcher
     if _launcher is None:
         from . import _launch as module
 
         lib = library()
         module.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
-                      for name in ("sr_cast", "sr_adamw_step", "sr_sgdm_step")))
+                      for name in ("sr_cast", "sr_adamw_step", "sr_sgdm_step", "sr_adamw_multi",
+                                   "sr_sgdm_multi")))
         _launcher = module
     return _launcher
 

@@ -35,20 +35,21 @@ def _launch(tables, dtypes, hparams, seed, rng_step, block_size, stream, row_sca
     ``row_scalars`` is None when every row shares ``hparams``, else a device
     tensor of per-row (neg_step_size, correction2_sqrt) FP32 pairs.
     """
-    _lib.call(
-        "sr_adamw_multi",
+    status = _lib.launcher().adamw_multi(
         tables.device_records.data_ptr(),
         tables.device_tile_rows.data_ptr(),
-        None if row_scalars is None else row_scalars.data_ptr(),
+        0 if row_scalars is None else row_scalars.data_ptr(),
         tables.nrows,
         tables.total_tiles,
         *dtypes,
-        ctypes.byref(hparams),
+        ctypes.addressof(hparams),
         seed,
         rng_step,
         block_size,
+        tables.device_records.get_device(),
         stream,
     )
+    _lib.check("sr_adamw_multi", status)
 
 
 def _validate_hyperparameters(lr, betas, eps, weight_decay):
@@ -59,7 +60,6 @@ def _validate_hyperparameters(lr, betas, eps, weight_decay):
         raise ValueError(f"invalid beta values: {betas}")
 
 
-@torch.no_grad()
 def hip_adamw_step_(
     parameter: torch.Tensor,
     gradient: torch.Tensor,
@@ -223,19 +223,19 @@ class AdamWHip(StateOptimizer):
 
         for launch in launches:
             dtypes = (*launch.codes, m_code, m_rule, v_code, v_rule)
-            with _lib.on_device(launch.device):
-                if isinstance(launch.steps, int):
-                    scalars, row_scalars = hparams(launch.steps), None
-                else:
-                    # Rows at different steps: each row's bias-correction pair.
-                    per_step = {step: hparams(step) for step in set(launch.steps)}
-                    pairs = np.array(
-                        [(per_step[s].neg_step_size, per_step[s].correction2_sqrt) for s in launch.steps],
-                        dtype=np.float32,
-                    )
+            if isinstance(launch.steps, int):
+                scalars, row_scalars = hparams(launch.steps), None
+            else:
+                # Rows at different steps: each row's bias-correction pair.
+                per_step = {step: hparams(step) for step in set(launch.steps)}
+                pairs = np.array(
+                    [(per_step[s].neg_step_size, per_step[s].correction2_sqrt) for s in launch.steps],
+                    dtype=np.float32,
+                )
+                with _lib.on_device(launch.device):
                     scalars, row_scalars = per_step[launch.steps[0]], upload(pairs, launch.device)
-                stream = _lib.stream_handle(launch.device)
-                _launch(launch.tables, dtypes, scalars, seed, rng_word, block_size, stream, row_scalars)
+            stream = _lib.stream_handle(launch.device)
+            _launch(launch.tables, dtypes, scalars, seed, rng_word, block_size, stream, row_scalars)
         record_steps()
 
 

@@ -32,14 +32,22 @@ def native_cast(x, *, dtype, rule, seed=0, offset=0, threads=_DEFAULT_THREADS, o
     if device.type != "cuda":
         raise ValueError(f"sr_states casts run on the GPU; got a {device.type} tensor")
     validate_device(device)
-    output = torch.empty_like(x, dtype=dtype, memory_format=torch.contiguous_format) if out is None else out
-    # The native entry checks `output` (dtype, shape, device, contiguity and
-    # no byte shared with x), then calls sr_cast with x's device current.
-    status = _lib.launcher().cast(x, output, _lib.DTYPE_CODES[dtype], rule, int(seed) & 0xFFFFFFFF,
-                                  int(offset) & 0xFFFFFFFF, threads, _lib.stream_handle(device))
+    launcher, code, stream = _lib.launcher(), _lib.DTYPE_CODES[dtype], _lib.stream_handle(device)
+    seed, offset = int(seed) & 0xFFFFFFFF, int(offset) & 0xFFFFFFFF
+    if out is None:
+        # Allocates natively; None for subclasses and __torch_function__ modes.
+        output = launcher.cast_new(x, code, rule, seed, offset, threads, stream)
+        if isinstance(output, torch.Tensor):
+            return output
+        if output is not None:
+            _lib.check("sr_cast", output)
+        out = torch.empty_like(x, dtype=dtype, memory_format=torch.contiguous_format)
+    # The native entry checks `out` (dtype, shape, device, contiguity and no
+    # byte shared with x), then calls sr_cast with x's device current.
+    status = launcher.cast(x, out, code, rule, seed, offset, threads, stream)
     if status:
         _lib.check("sr_cast", status)
-    return output
+    return out
 
 
 NEIGHBOR_DTYPES = (torch.bfloat16, torch.float16, torch.float8_e4m3fn, torch.float8_e5m2)

@@ -29,22 +29,22 @@ _STATE_NAMES = ("momentum_buffer",)
 
 def _launch(tables, dtypes, hparams, seed, rng_step, block_size, stream):
     """One sr_sgdm_multi call; dtypes = (p, g, u, u_rule) codes."""
-    _lib.call(
-        "sr_sgdm_multi",
+    status = _lib.launcher().sgdm_multi(
         tables.device_records.data_ptr(),
         tables.device_tile_rows.data_ptr(),
         tables.nrows,
         tables.total_tiles,
         *dtypes,
-        ctypes.byref(hparams),
+        ctypes.addressof(hparams),
         seed,
         rng_step,
         block_size,
+        tables.device_records.get_device(),
         stream,
     )
+    _lib.check("sr_sgdm_multi", status)
 
 
-@torch.no_grad()
 def hip_sgdm_step_(
     parameter: torch.Tensor,
     gradient: torch.Tensor,
@@ -165,16 +165,15 @@ class SGDMHip(StateOptimizer):
         seed, rng_word = _lib.low64(group["sr_seed"]), _lib.low64(rng_step)
         block_size = self._group_block_size(group)
         for launch in launches:
-            with _lib.on_device(launch.device):
-                _launch(
-                    launch.tables,
-                    (*launch.codes, code, rule),
-                    hparams,
-                    seed,
-                    rng_word,
-                    block_size,
-                    _lib.stream_handle(launch.device),
-                )
+            _launch(
+                launch.tables,
+                (*launch.codes, code, rule),
+                hparams,
+                seed,
+                rng_word,
+                block_size,
+                _lib.stream_handle(launch.device),
+            )
         record_steps()
 
 

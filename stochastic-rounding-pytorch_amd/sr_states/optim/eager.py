@@ -31,8 +31,7 @@ reference's lazy loop does (sr_states/optim/_state.py:154-182).
 
 from __future__ import annotations
 
-import torch
-
+from .. import _lib
 from ..hip._common import validate_update_device
 from ..hip._multi_tensor import prepare_group
 from ..hip._optimizer import DEFAULT_BLOCK_SIZE
@@ -73,7 +72,7 @@ class _FusedGroups(StateOptimizer):
         """The fused launches of the group, or None to update it per parameter."""
         if not self._fused_route or not all(has_native(f.dtype, f.rounding) for f in formats):
             return None
-        if torch.cuda.is_available() and torch.cuda.is_current_stream_capturing():
+        if _lib.capturing():
             return None
         try:
             self._validate_group(group)

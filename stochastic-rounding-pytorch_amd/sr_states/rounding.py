@@ -125,17 +125,21 @@ def cast(
     return result
 
 
+_native_cast = None
+
+
 def _builtin(code: int, rule: int) -> Callable:
     if code == _lib.SR_F32:
         def routine(x, *, dtype, seed, offset):
             return x
     else:
         def routine(x, *, dtype, seed, offset):
-            # Imported here: sr_states.hip imports this module.
-            from .hip.cast import native_cast
-
-            return native_cast(x if x.is_contiguous() else x.contiguous(), dtype=dtype, rule=rule,
-                               seed=seed, offset=offset)
+            global _native_cast
+            if _native_cast is None:
+                # Imported at the first cast: sr_states.hip imports this module.
+                from .hip.cast import native_cast as _native_cast
+            return _native_cast(x if x.is_contiguous() else x.contiguous(), dtype=dtype, rule=rule,
+                                seed=seed, offset=offset)
 
     routine.__name__ = f"hip_cast_{code}_{rule}"
     return routine
