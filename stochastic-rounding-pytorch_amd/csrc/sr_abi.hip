@@ -82,15 +82,17 @@ int param_enc(int index) { return index == 0 ? sr::ENC_F32 : sr::ENC_BF16_RN; }
 
 bool valid_block(int block) { return block >= 64 && block <= sr::kMaxBlock && block % 64 == 0; }
 
-// One workgroup per tile; the grid is padded to a whole number of XCD chunk
-// rounds so that the kernels' tile order (sr_tile_order.h) is a permutation,
-// and split into rows when one dimension would carry 2^32 or more
-// work-items (2^34 elements at four per lane).  `tiles` must equal the
-// total_tiles the kernel argument carries.  `cap` > 0 limits the resident
-// workgroups per CU to that many (sr::cap_lds).
-int launch(const void* fn, int block, uint32_t tiles, void* arg, void* stream, uint32_t cap = 0) {
+// One workgroup per tile.  In the chunked order the grid is padded to a whole
+// number of XCD chunk rounds so that the order (sr_tile_order.h) is a
+// permutation; either grid is split into rows when one dimension would carry
+// 2^32 or more work-items (2^34 elements at four per lane).  `tiles` and
+// `in_sequence` must equal what the kernel argument carries.  `cap` > 0
+// limits the resident workgroups per CU to that many (sr::cap_lds).
+int launch(const void* fn, int block, uint32_t tiles, void* arg, void* stream, bool in_sequence = false,
+           uint32_t cap = 0) {
   if (sr::padded_grid(tiles) > 0x7FFFFFFFull) return fail(SR_ERR_ARGUMENT, "%u tiles exceed the grid limit", tiles);
-  const sr::LaunchShape shape = sr::launch_shape(tiles, static_cast<uint32_t>(block));
+  const sr::LaunchShape shape = in_sequence ? sr::sequence_shape(tiles, static_cast<uint32_t>(block))
+                                            : sr::launch_shape(tiles, static_cast<uint32_t>(block));
   void* args[] = {arg};
   hipError_t err = hipLaunchKernel(fn, dim3(shape.x, shape.y), dim3(block), args, sr::cap_lds(fn, block, cap),
                                    static_cast<hipStream_t>(stream));
@@ -99,7 +101,7 @@ int launch(const void* fn, int block, uint32_t tiles, void* arg, void* stream, u
 }
 
 // SR_STATES_RESIDENT_CAP, read once (sr::resident_cap_override): the cap of
-// every launch of at least 2^16 tiles, or -1 for the rule.
+// every launch of at least 2^16 tiles or in sequence, or -1 for the rules.
 int cap_override() {
   static const int value = sr::resident_cap_override(std::getenv("SR_STATES_RESIDENT_CAP"));
   return value;
@@ -108,24 +110,39 @@ int cap_override() {
 // Whether an encoding rounds stochastically to FP16 or FP8.
 bool minifloat_sr(int enc) { return enc == sr::ENC_F16_SR || enc == sr::ENC_E4M3_SR || enc == sr::ENC_E5M2_SR; }
 
-// Resident-workgroup cap of an AdamW launch (sr::resident_cap).
-uint32_t adamw_cap(int pi, int gi, int me, int ve, int block, uint32_t tiles) {
-  if (cap_override() >= 0) return tiles >= sr::kResidentCapMinTiles ? static_cast<uint32_t>(cap_override()) : 0u;
-  const int bytes = 2 * sr::enc_bytes(param_enc(pi)) + sr::enc_bytes(param_enc(gi)) + 2 * sr::enc_bytes(me) +
-                    2 * sr::enc_bytes(ve);
-  const uint32_t in_flight = sr::adamw_in_flight(gi == 1, minifloat_sr(me) && minifloat_sr(ve));
-  return sr::resident_cap(tiles, static_cast<uint32_t>(block),
-                          static_cast<uint32_t>(sr::lane_elements(param_enc(pi), param_enc(gi), me, ve)),
-                          static_cast<uint32_t>(bytes), pi == 0, in_flight);
+// Launches an optimizer kernel over a.total_tiles tiles of block * lanes
+// elements in the order its size and operands ask for, with that order's cap
+// on the resident workgroups.  `chunked_in_flight` is the chunked order's
+// budget, `moments_sr` how many of the `moments` are minifloat_sr.
+template <class Args>
+int launch_update(const void* fn, Args& a, int block, int lanes, bool bf16_params, bool bf16_gradient,
+                  uint32_t moments, uint32_t moments_sr, uint32_t bytes, uint32_t chunked_in_flight, void* stream) {
+  const uint32_t tiles = a.total_tiles, b = static_cast<uint32_t>(block), l = static_cast<uint32_t>(lanes);
+  a.in_sequence = sr::use_sequence(tiles, b, l, bf16_params, bf16_gradient, moments, moments_sr, bytes);
+  uint32_t cap;
+  if (cap_override() >= 0) {
+    cap = a.in_sequence || tiles >= sr::kResidentCapMinTiles ? static_cast<uint32_t>(cap_override()) : 0u;
+  } else if (a.in_sequence) {
+    cap = sr::workgroups_in(sr::sequence_in_flight(moments_sr), b, l, bytes);
+  } else {
+    cap = sr::resident_cap(tiles, b, l, bytes, !bf16_params, chunked_in_flight);
+  }
+  return launch(fn, block, tiles, &a, stream, a.in_sequence, cap);
 }
 
-// Resident-workgroup cap of a momentum-SGD launch.
-uint32_t sgdm_cap(int pi, int gi, int ue, int block, uint32_t tiles) {
-  if (cap_override() >= 0) return tiles >= sr::kResidentCapMinTiles ? static_cast<uint32_t>(cap_override()) : 0u;
-  const int bytes = 2 * sr::enc_bytes(param_enc(pi)) + sr::enc_bytes(param_enc(gi)) + 2 * sr::enc_bytes(ue);
-  return sr::resident_cap(tiles, static_cast<uint32_t>(block),
-                          static_cast<uint32_t>(sr::lane_elements(param_enc(pi), param_enc(gi), ue, ue)),
-                          static_cast<uint32_t>(bytes), pi == 0, sr::sgdm_in_flight(ue == sr::ENC_F16_SR));
+int launch_adamw(sr::AdamWArgs& a, int pi, int gi, int me, int ve, int block, void* stream) {
+  const uint32_t bytes = 2 * sr::enc_bytes(param_enc(pi)) + sr::enc_bytes(param_enc(gi)) + 2 * sr::enc_bytes(me) +
+                         2 * sr::enc_bytes(ve);
+  return launch_update(tables().adamw[pi][gi][me][ve], a, block,
+                       sr::lane_elements(param_enc(pi), param_enc(gi), me, ve), pi == 1, gi == 1, 2,
+                       static_cast<uint32_t>(minifloat_sr(me)) + minifloat_sr(ve), bytes,
+                       sr::adamw_in_flight(gi == 1, minifloat_sr(me) && minifloat_sr(ve)), stream);
+}
+
+int launch_sgdm(sr::SgdmArgs& a, int pi, int gi, int ue, int block, void* stream) {
+  const uint32_t bytes = 2 * sr::enc_bytes(param_enc(pi)) + sr::enc_bytes(param_enc(gi)) + 2 * sr::enc_bytes(ue);
+  return launch_update(tables().sgdm[pi][gi][ue], a, block, sr::lane_elements(param_enc(pi), param_enc(gi), ue, ue),
+                       pi == 1, gi == 1, 1, minifloat_sr(ue), bytes, sr::sgdm_in_flight(ue == sr::ENC_F16_SR), stream);
 }
 
 // Tiles of block * lanes elements covering n elements, or fail if they do
@@ -356,8 +373,7 @@ int sr_adamw_step(void* p, const void* g, void* m, void* v, int64_t n, int p_dty
   r.param_index = key;
   r.shard_start = offset;
   r.flags = SR_ROW_KEYED;
-  return launch(tables().adamw[pi][gi][me][ve], block_size, a.total_tiles, &a, stream,
-                adamw_cap(pi, gi, me, ve, block_size, a.total_tiles));
+  return launch_adamw(a, pi, gi, me, ve, block_size, stream);
 }
 
 int sr_adamw_multi(const sr_row* rows, const uint32_t* tile_rows, const float* row_scalars,
@@ -384,8 +400,7 @@ int sr_adamw_multi(const sr_row* rows, const uint32_t* tile_rows, const float* r
   a.key_prefix = sr::update_key_prefix(static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32),
                                        static_cast<uint32_t>(rng_step),
                                        static_cast<uint32_t>(rng_step >> 32));
-  return launch(tables().adamw[pi][gi][me][ve], block_size, total_tiles, &a, stream,
-                adamw_cap(pi, gi, me, ve, block_size, total_tiles));
+  return launch_adamw(a, pi, gi, me, ve, block_size, stream);
 }
 
 int sr_sgdm_step(void* p, const void* g, void* u, int64_t n, int p_dtype, int g_dtype, int u_dtype,
@@ -417,8 +432,7 @@ int sr_sgdm_step(void* p, const void* g, void* u, int64_t n, int p_dtype, int g_
   r.param_index = key;
   r.shard_start = offset;
   r.flags = SR_ROW_KEYED;
-  return launch(tables().sgdm[pi][gi][ue], block_size, a.total_tiles, &a, stream,
-                sgdm_cap(pi, gi, ue, block_size, a.total_tiles));
+  return launch_sgdm(a, pi, gi, ue, block_size, stream);
 }
 
 int sr_sgdm_multi(const sr_row* rows, const uint32_t* tile_rows, int nrows, uint32_t total_tiles,
@@ -441,8 +455,7 @@ int sr_sgdm_multi(const sr_row* rows, const uint32_t* tile_rows, int nrows, uint
   a.key_prefix = sr::update_key_prefix(static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32),
                                        static_cast<uint32_t>(rng_step),
                                        static_cast<uint32_t>(rng_step >> 32));
-  return launch(tables().sgdm[pi][gi][ue], block_size, total_tiles, &a, stream,
-                sgdm_cap(pi, gi, ue, block_size, total_tiles));
+  return launch_sgdm(a, pi, gi, ue, block_size, stream);
 }
 
 int sr_adamw_multi_noalloc(const sr_row* rows, const float* row_scalars, int nrows, uint32_t total_tiles,
@@ -493,8 +506,7 @@ int sr_adamw_multi_noalloc(const sr_row* rows, const float* row_scalars, int nro
   a.key_prefix = sr::update_key_prefix(static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32),
                                        static_cast<uint32_t>(rng_step),
                                        static_cast<uint32_t>(rng_step >> 32));
-  return launch(tables().adamw[pi][gi][me][ve], block_size, total_tiles, &a, stream,
-                adamw_cap(pi, gi, me, ve, block_size, total_tiles));
+  return launch_adamw(a, pi, gi, me, ve, block_size, stream);
 }
 
 }  // extern "C"

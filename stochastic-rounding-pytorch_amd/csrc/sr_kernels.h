@@ -16,11 +16,11 @@
 // BF16 with E5M2-SR m, 13 M 38.8 -> 32.5.  The partial last tile of a row
 // takes whole groups too, and its last lanes the 1-3 elements after them.
 //
-// XCD-aware order.  Workgroups map to tiles through sr_tile_order.h: each
-// XCD takes chunks of up to 512 consecutive tiles in turn, so the tiles in
-// flight on one XCD stay close together.  Measured on MI355X for the
-// 12-byte-read / 8-byte-write pattern of the fused update, this order and one
-// tile per workgroup beat persistent grid-stride loops.
+// Tile order (sr_tile_order.h).  Large optimizer launches with much arithmetic
+// per byte take their tiles in sequence, so that what is in flight on the
+// whole chip is one window per stream; all others deal chunks of up to 512
+// consecutive tiles to the XCDs in turn.  Either order with one tile per
+// workgroup beat persistent grid-stride loops.
 //
 // Multi-tensor launches.  `tile_rows[t]` names the row (tensor) of tile t
 // and `rows[row]` is its 64-byte sr_row record: both are read once per
@@ -57,6 +57,7 @@ struct AdamWArgs {
   AdamWScalars s;
   uint32_t total_tiles;
   uint32_t key_prefix;  // update_key_prefix(seed, rng_step), computed by the host
+  uint32_t in_sequence;  // workgroup b takes tile b; else the chunked order
 };
 
 struct SgdmArgs {
@@ -66,6 +67,7 @@ struct SgdmArgs {
   SgdmScalars s;
   uint32_t total_tiles;
   uint32_t key_prefix;  // update_key_prefix(seed, rng_step), computed by the host
+  uint32_t in_sequence;  // workgroup b takes tile b; else the chunked order
 };
 
 struct CastArgs {
@@ -77,11 +79,12 @@ struct CastArgs {
 };
 
 // Logical tile of this workgroup; >= total_tiles for the padding workgroups.
-// The host launches launch_shape(total_tiles, block): one row of
-// padded_grid(total_tiles) workgroups, or several rows when that many would
-// exceed the dispatch packet's 32-bit work-item count.
-__device__ __forceinline__ uint32_t logical_tile(uint32_t total_tiles) {
-  return tile_of(blockIdx.y * gridDim.x + blockIdx.x, total_tiles);
+// The host launches sequence_shape(total_tiles, block) or launch_shape(...):
+// one row of workgroups, or several rows when that many would exceed the
+// dispatch packet's 32-bit work-item count.
+__device__ __forceinline__ uint32_t logical_tile(uint32_t total_tiles, bool in_sequence = false) {
+  const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
+  return in_sequence ? b : tile_of(b, total_tiles);
 }
 
 // ---------------------------------------------------------------------------
@@ -314,7 +317,7 @@ __device__ __forceinline__ void adamw_scalar(char* p, const char* g, char* m, ch
 template <int PE, int GE, int ME, int VE>
 __global__ __launch_bounds__(kMaxBlock) void adamw_kernel(const AdamWArgs a) {
   constexpr int E = lane_elements(PE, GE, ME, VE);
-  const uint32_t t = logical_tile(a.total_tiles);
+  const uint32_t t = logical_tile(a.total_tiles, a.in_sequence);
   if (t >= a.total_tiles) return;
   const uint32_t row = tile_row_index(a, t);
   const sr_row r = row_record(a, row);
@@ -382,7 +385,7 @@ __device__ __forceinline__ void sgdm_scalar(char* p, const char* g, char* u, int
 template <int PE, int GE, int UE>
 __global__ __launch_bounds__(kMaxBlock) void sgdm_kernel(const SgdmArgs a) {
   constexpr int E = lane_elements(PE, GE, UE, UE);
-  const uint32_t t = logical_tile(a.total_tiles);
+  const uint32_t t = logical_tile(a.total_tiles, a.in_sequence);
   if (t >= a.total_tiles) return;
   const sr_row r = row_record(a, tile_row_index(a, t));
   char* p = reinterpret_cast<char*>(r.ptr[0]);

@@ -2,19 +2,21 @@
 //
 // Shared by the kernels and by the host code that sizes the grid, and plain
 // C++ otherwise, so it also compiles on the host alone.  It also holds the
-// rule for how many workgroups of a large optimizer launch stay resident
-// per CU (resident_cap, at the end).
+// rules for how many workgroups of a large optimizer launch stay resident
+// per CU, with each order's own budgets (at the end).
 //
-// The dispatcher hands workgroup b to XCD (b mod 8).  Tiles are dealt to the
+// Two orders.  Large optimizer launches with much arithmetic per byte take
+// their tiles in sequence, workgroup b tile b (use_sequence below); every
+// other launch takes the chunked order that follows.
+//
+// Chunked order.  The dispatcher hands workgroup b to XCD (b mod 8).  Tiles are dealt to the
 // XCDs in chunks of 2^s consecutive tiles: XCD x takes chunks x, x + 8,
 // x + 16, ..., and its k-th workgroup takes tile (k mod 2^s) of its
 // (k >> s)-th chunk.  The tiles in flight on one XCD therefore stay within a
 // few neighbouring chunks, and the eight XCDs stream eight neighbouring
 // chunks.  s is at most 9 (512-tile chunks) and small enough that 64 chunks
 // fit in the launch, so padding the grid to a multiple of 8 chunks adds less
-// than one eighth of it.  Measured on MI355X for the fused update's
-// 12-byte-read / 8-byte-write pattern, 512-tile chunks beat both plain order
-// and one contiguous eighth of the tiles per XCD.
+// than one eighth of it.
 #pragma once
 
 #include <cstdint>
@@ -75,8 +77,57 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
   return {static_cast<uint32_t>(per_row), static_cast<uint32_t>((grid + per_row - 1) / per_row)};
 }
 
-// Resident workgroups per CU of a large optimizer launch.  The fused updates
-// use few registers, so 16 of their 128-lane workgroups fit on a CU, and
+// Sequential order.  With workgroup b on tile b, what is in flight on the
+// chip is one window per stream, a few MiB wide; the chunked order has eight,
+// one an XCD.  HBM serves several streams the worse the wider the addresses in
+// flight spread, and the more of them there are (the caps below).  Launches
+// whose workgroups live long need many in flight, so there the narrower
+// window pays.  Their tile-map entries come from more cache lines, since
+// neighbouring tiles run on different XCDs, which is why launches of FP32
+// parameters and gradients with cheap or wide moments stay chunked: in
+// sequence they measured 0 to 2% less (BF16-SR moments, 1.55 * 10^9 elements:
+// 4.85 against 4.79 ms; FP32 moments, 7.4 * 10^8: 6.21 against 6.36 TB/s).
+//
+// MI355X, 24 tensors, mean over 6 placements, TB/s, chunked at its own best
+// cap -> in sequence at its best, at 2.6 * 10^8 and 7.4 * 10^8 elements:
+// BF16 p/g with BF16-SR m/v 6.42 -> 6.53 and 6.29 -> 6.51, BF16-nearest 6.31
+// -> 6.59 and 6.23 -> 6.58, FP32 6.14 -> 6.47 and 6.10 -> 6.39, E4M3-SR m 6.12
+// -> 6.31 and 6.13 -> 6.26, FP16-SR 6.14 -> 6.33 and 6.14 -> 6.25; FP32 p with
+// BF16 g and BF16-SR m/v 6.39 -> 6.58 and 6.30 -> 6.56, FP8-nearest 6.44 -> 6.56
+// and 6.32 -> 6.54 (1.3 and 5 * 10^8), FP16-SR 6.40 -> 6.45 and 6.23 -> 6.39;
+// FP32 p/g with E4M3-SR m 6.45 -> 6.57 and 6.36 -> 6.50.  SGDM with BF16 p/g
+// and FP32 momentum 6.51 -> 6.62, E4M3-SR 6.53 -> 6.80, with BF16 g 6.58 -> 6.63.
+// Level or worse, hence chunked: FP32 p/g with two FP8-SR moments (-1.3 to
+// +0.5%) or two FP16-SR ones (-0.6 to +1%), SGDM with FP32 p/g (-0.9%), and
+// SGDM with BF16 p/g and BF16 momentum (10 B: -2.5 to 0%).
+//
+// From 5 * 2^21 elements on; below, the chunked order is level or better.
+constexpr uint64_t kSequenceMinElements = 5ull << 21;
+
+// `moments` is 2 for AdamW and 1 for SGDM, `minifloat_sr` counts the moments
+// that round stochastically to FP16 or FP8.
+SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params,
+                                        bool bf16_gradient, uint32_t moments, uint32_t minifloat_sr,
+                                        uint32_t bytes_per_element) {
+  const bool long_lived = bf16_params     ? moments == 2 || minifloat_sr > 0 || bytes_per_element >= 14
+                          : bf16_gradient ? bytes_per_element <= 18
+                                          : minifloat_sr == 1 && bytes_per_element >= 18 && bytes_per_element <= 20;
+  return long_lived && static_cast<uint64_t>(tiles) * block * lanes >= kSequenceMinElements;
+}
+
+// Grid of a launch in sequence: `tiles` workgroups, in rows where one
+// dimension cannot hold them (launch_shape); workgroups past the last tile
+// leave at once.
+SR_HOST_DEVICE inline LaunchShape sequence_shape(uint32_t tiles, uint32_t block,
+                                                 uint64_t max_items = 0xFFFFFFFFull) {
+  const uint64_t per_row = max_items / block;
+  if (tiles <= per_row) return {tiles, 1u};
+  return {static_cast<uint32_t>(per_row), static_cast<uint32_t>((tiles + per_row - 1) / per_row)};
+}
+
+// Resident workgroups per CU of a large optimizer launch in the chunked
+// order (those in sequence: sequence_in_flight).  The fused updates use few
+// registers, so 16 of their 128-lane workgroups fit on a CU, and
 // that many keep more memory requests in flight than HBM can serve: the
 // surplus only adds contention.  The cap is round(budget / tile bytes), the
 // budget being the bytes of tiles in flight per CU at which the rate peaked
@@ -101,11 +152,10 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
 //     6.47-6.49 at 11; FP32: 6.21 -> 6.43 at 9; FP8: best at 12-13), except
 //     FP16-SR momentum at 72 KiB (6.35-6.38 -> 6.58-6.61 at 9, against
 //     6.50-6.54 at 10 and 6.48 at 11, on three machines).
-// Launches with BF16 parameters spend more of a workgroup's life in
-// arithmetic; caps of 11 to 15 moved them by under 1%, so they stay
-// uncapped, as do launches of fewer than 2^16 tiles (2^25 elements at 128
-// lanes), whose tail the cap lengthens (2^24 elements: 6.50 -> 6.46;
-// 2^25: 6.53 -> 6.62), and the casts (every cap slower).  A budget that
+// In this order launches with BF16 parameters gain nothing from a cap, and
+// launches of fewer than 2^16 tiles (2^25 elements at 128 lanes), whose tail
+// the cap lengthens (2^24 elements: 6.50 -> 6.46; 2^25: 6.53 -> 6.62), and the
+// casts (every cap slower) have none.  A budget that
 // rounds to more than kResidentCapMax workgroups also means no cap.
 constexpr uint32_t kInFlightAdamW = 80u * 1024u;
 constexpr uint32_t kInFlightAdamWWide = 96u * 1024u;
@@ -125,6 +175,16 @@ SR_HOST_DEVICE constexpr uint32_t sgdm_in_flight(bool f16_sr_momentum) {
   return f16_sr_momentum ? kInFlightSgdmF16Sr : kInFlightSgdm;
 }
 
+// Workgroups whose tiles hold `in_flight` bytes, rounded, or 0 (no cap) where
+// that is none or more than kResidentCapMax.
+SR_HOST_DEVICE inline uint32_t workgroups_in(uint32_t in_flight, uint32_t block, uint32_t lanes,
+                                             uint32_t bytes_per_element) {
+  const uint64_t tile_bytes = static_cast<uint64_t>(block) * lanes * bytes_per_element;
+  if (tile_bytes == 0) return 0;
+  const uint64_t cap = (in_flight + tile_bytes / 2) / tile_bytes;
+  return cap >= 1 && cap <= kResidentCapMax ? static_cast<uint32_t>(cap) : 0u;
+}
+
 // Workgroups per CU to leave resident for an optimizer launch of `tiles`
 // tiles of `block` lanes times `lanes` elements, moving `bytes_per_element`
 // bytes per element with `in_flight` bytes of tiles in flight per CU, or 0
@@ -133,14 +193,24 @@ SR_HOST_DEVICE inline uint32_t resident_cap(uint32_t tiles, uint32_t block, uint
                                             uint32_t bytes_per_element, bool fp32_params,
                                             uint32_t in_flight = kInFlightAdamW) {
   if (!fp32_params || tiles < kResidentCapMinTiles) return 0;
-  const uint64_t tile_bytes = static_cast<uint64_t>(block) * lanes * bytes_per_element;
-  if (tile_bytes == 0) return 0;
-  const uint64_t cap = (in_flight + tile_bytes / 2) / tile_bytes;
-  return cap >= 1 && cap <= kResidentCapMax ? static_cast<uint32_t>(cap) : 0u;
+  return workgroups_in(in_flight, block, lanes, bytes_per_element);
+}
+
+// Bytes of tiles in flight per CU of a launch in sequence, where the rate
+// peaked on MI355X over 26 combinations of operand types (caps 5 to 14 and
+// none, as above): 88 KiB, 96 with one moment that rounds stochastically to
+// FP16 or FP8, 104 with two; a cap past kResidentCapMax means none, as in the
+// chunked order.  The caps this gives, best measured in parentheses: BF16 p/g
+// with BF16-SR m/v 13 (12-13, which reserve alike), BF16-nearest 13 (11-12),
+// FP32 8 (7-9), E4M3-SR m none (none), FP16-SR none (none); BF16 g with BF16-SR
+// 10 (9-10), FP8-nearest 13 (12), E4M3-SR m 12 (12-14), FP16-SR m 11 (10-11),
+// two FP16-SR 12 (11-12), two E4M3-SR none (none); FP32 p/g with E4M3-SR m 11 (10-11).
+SR_HOST_DEVICE constexpr uint32_t sequence_in_flight(uint32_t minifloat_sr) {
+  return (88u + 8u * minifloat_sr) * 1024u;
 }
 
 // The environment can replace the rule: SR_STATES_RESIDENT_CAP=k caps every
-// optimizer launch of at least 2^16 tiles (any parameter dtype) at k
+// optimizer launch of at least 2^16 tiles, and every one in sequence, at k
 // workgroups per CU, 1 <= k <= kResidentCapOverrideMax, and 0 leaves them
 // all uncapped.  For measuring the rule and for workloads whose best cap
 // differs; results never depend on it.  resident_cap_override parses the

@@ -1,0 +1,53 @@
+// Checks the grid of launches in sequence (csrc/sr_tile_order.h) on the host:
+// sequence_shape covers every tile exactly once, each dimension within its
+// work-item limit and fewer than one row of padding, and workgroup numbers
+// stay within 32 bits; use_sequence starts at its element count for every
+// workgroup size; workgroups_in keeps within its largest cap.
+#include <cstdint>
+#include <cstdio>
+#include <initializer_list>
+
+#include "sr_tile_order.h"
+
+int main() {
+  int failures = 0, shapes = 0;
+  for (uint32_t tiles : {1u, 63u, 20480u, 33554431u, 33554432u, 33556480u, 0x7FFFF000u}) {
+    for (uint32_t block : {64u, 128u, 256u, 512u, 1024u}) {
+      for (uint64_t limit : {1ull << 16, 1ull << 24, 0xFFFFFFFFull}) {
+        const sr::LaunchShape shape = sr::sequence_shape(tiles, block, limit);
+        const uint64_t total = static_cast<uint64_t>(shape.x) * shape.y;
+        ++shapes;
+        // Workgroup b takes tile b, so covering [0, tiles) is total >= tiles.
+        if (total < tiles || total - tiles >= shape.x || static_cast<uint64_t>(shape.x) * block > limit ||
+            total >= (1ull << 32)) {
+          std::printf("tiles %u block %u limit %llu: %u x %u\n", tiles, block, (unsigned long long)limit, shape.x,
+                      shape.y);
+          ++failures;
+        }
+      }
+    }
+  }
+  for (uint32_t block : {128u, 256u, 512u, 1024u}) {
+    const uint32_t edge = static_cast<uint32_t>(sr::kSequenceMinElements / (block * 4));
+    if (!sr::use_sequence(edge, block, 4, true, true, 2, 0, 14) ||
+        sr::use_sequence(edge - 1, block, 4, true, true, 2, 0, 14) ||
+        sr::use_sequence(edge, block, 4, false, false, 2, 0, 20)) {
+      std::printf("block %u: the rule's edge moved\n", block);
+      ++failures;
+    }
+  }
+  for (uint32_t bytes = 6; bytes <= 28; ++bytes) {
+    for (uint32_t block : {64u, 128u, 1024u}) {
+      for (uint32_t moments : {0u, 1u, 2u}) {
+        const uint32_t budget = sr::sequence_in_flight(moments), cap = sr::workgroups_in(budget, block, 4, bytes);
+        const uint32_t tile = block * 4 * bytes;
+        if (cap > sr::kResidentCapMax || (cap && (2 * cap * tile > 2 * budget + tile || 2 * (cap + 1) * tile < 2 * budget))) {
+          std::printf("cap %u for %u bytes, block %u, budget %u\n", cap, bytes, block, budget);
+          ++failures;
+        }
+      }
+    }
+  }
+  std::printf("%d shapes, %d failures\n", shapes, failures);
+  return failures != 0;
+}

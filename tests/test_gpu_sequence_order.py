@@ -1,0 +1,54 @@
+"""Launches on both sides of the tile-order rule against the C oracle, byte for byte.
+
+From 5 * 2^21 elements on, launches with BF16 parameters take their tiles in
+sequence with a cap on the resident workgroups; one tile fewer, the chunked
+order.  The element count ends in a partial tile with a remainder, and the
+group spreads it over three tensors, one of which starts off 16-byte
+alignment.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import c_oracle, sr_oracle
+
+pytestmark = pytest.mark.gpu
+
+EDGE = 5 << 21
+BF16, F16, E4M3 = torch.bfloat16, torch.float16, torch.float8_e4m3fn
+
+
+@pytest.mark.parametrize("block_size", (128, 512))
+@pytest.mark.parametrize("total", (EDGE - 4 * 512 - 1, EDGE + 3))
+@pytest.mark.parametrize("moments", [(BF16, BF16), (F16, E4M3)])
+def test_both_sides_of_the_order_rule_equal_the_oracle(cuda, moments, total, block_size):
+    import sr_states
+
+    formats = tuple((dtype, "stochastic") for dtype in moments)
+    sizes = (1021, 4 * 1024 * 1024 + 1, total - 1021 - 4 * 1024 * 1024 - 1)
+    generator = torch.Generator().manual_seed(total)
+    params, grads = [], []
+    for n in sizes:
+        params.append(torch.randn(n, generator=generator).to(BF16))
+        grads.append((torch.randn(n, generator=generator) * 0.1).to(BF16))
+    flat = torch.zeros(total + 1, dtype=BF16, device=cuda)
+    start, views = 1, []
+    for n, g in zip(sizes, grads):
+        views.append(flat[start:start + n].copy_(g))
+        start += n
+    device = [torch.nn.Parameter(p.to(cuda)) for p in params]
+    optimizer = sr_states.AdamWHip(
+        device, lr=3e-4, weight_decay=0.01, seed=7, block_size=block_size,
+        state_format={name: sr_states.StateFormat(*f) for name, f in zip(("exp_avg", "exp_avg_sq"), formats)})
+    for p, g in zip(device, views):
+        p.grad = g
+    optimizer.step()
+    for index, (p, g, got) in enumerate(zip(params, grads, device)):
+        m, v = (torch.zeros(p.shape, dtype=dtype) for dtype in moments)
+        c_oracle.adamw_step_(p, g, m, v, lr=3e-4, beta1=0.9, beta2=0.999, eps=1e-8, weight_decay=0.01, step=1,
+                             formats=formats, seed=sr_oracle.update_key(7, 1, index))
+        state = optimizer.state[got]
+        for have, want in ((got.detach(), p), (state["exp_avg"], m), (state["exp_avg_sq"], v)):
+            assert torch.equal(have.cpu().view(torch.uint8), want.view(torch.uint8)), (index, total, moments)
