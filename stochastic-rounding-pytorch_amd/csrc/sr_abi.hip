@@ -115,10 +115,10 @@ bool minifloat_sr(int enc) { return enc == sr::ENC_F16_SR || enc == sr::ENC_E4M3
 // on the resident workgroups.  `chunked_in_flight` is the chunked order's
 // budget, `moments_sr` how many of the `moments` are minifloat_sr.
 template <class Args>
-int launch_update(const void* fn, Args& a, int block, int lanes, bool bf16_params, bool bf16_gradient,
-                  uint32_t moments, uint32_t moments_sr, uint32_t bytes, uint32_t chunked_in_flight, void* stream) {
+int launch_update(const void* fn, Args& a, int block, int lanes, bool bf16_params, uint32_t moments,
+                  uint32_t moments_sr, uint32_t bytes, uint32_t chunked_in_flight, void* stream) {
   const uint32_t tiles = a.total_tiles, b = static_cast<uint32_t>(block), l = static_cast<uint32_t>(lanes);
-  a.in_sequence = sr::use_sequence(tiles, b, l, bf16_params, bf16_gradient, moments, moments_sr, bytes);
+  a.in_sequence = sr::use_sequence(tiles, b, l, bf16_params, moments, moments_sr, bytes);
   uint32_t cap;
   if (cap_override() >= 0) {
     cap = a.in_sequence || tiles >= sr::kResidentCapMinTiles ? static_cast<uint32_t>(cap_override()) : 0u;
@@ -134,7 +134,7 @@ int launch_adamw(sr::AdamWArgs& a, int pi, int gi, int me, int ve, int block, vo
   const uint32_t bytes = 2 * sr::enc_bytes(param_enc(pi)) + sr::enc_bytes(param_enc(gi)) + 2 * sr::enc_bytes(me) +
                          2 * sr::enc_bytes(ve);
   return launch_update(tables().adamw[pi][gi][me][ve], a, block,
-                       sr::lane_elements(param_enc(pi), param_enc(gi), me, ve), pi == 1, gi == 1, 2,
+                       sr::lane_elements(param_enc(pi), param_enc(gi), me, ve), pi == 1, 2,
                        static_cast<uint32_t>(minifloat_sr(me)) + minifloat_sr(ve), bytes,
                        sr::adamw_in_flight(gi == 1, minifloat_sr(me) && minifloat_sr(ve)), stream);
 }
@@ -142,7 +142,7 @@ int launch_adamw(sr::AdamWArgs& a, int pi, int gi, int me, int ve, int block, vo
 int launch_sgdm(sr::SgdmArgs& a, int pi, int gi, int ue, int block, void* stream) {
   const uint32_t bytes = 2 * sr::enc_bytes(param_enc(pi)) + sr::enc_bytes(param_enc(gi)) + 2 * sr::enc_bytes(ue);
   return launch_update(tables().sgdm[pi][gi][ue], a, block, sr::lane_elements(param_enc(pi), param_enc(gi), ue, ue),
-                       pi == 1, gi == 1, 1, minifloat_sr(ue), bytes, sr::sgdm_in_flight(ue == sr::ENC_F16_SR), stream);
+                       pi == 1, 1, minifloat_sr(ue), bytes, sr::sgdm_in_flight(ue == sr::ENC_F16_SR), stream);
 }
 
 // Tiles of block * lanes elements covering n elements, or fail if they do

@@ -16,8 +16,8 @@
 // BF16 with E5M2-SR m, 13 M 38.8 -> 32.5.  The partial last tile of a row
 // takes whole groups too, and its last lanes the 1-3 elements after them.
 //
-// Tile order (sr_tile_order.h).  Large optimizer launches with much arithmetic
-// per byte take their tiles in sequence, so that what is in flight on the
+// Tile order (sr_tile_order.h).  Large optimizer launches with BF16 parameters
+// take their tiles in sequence, so that what is in flight on the
 // whole chip is one window per stream; all others deal chunks of up to 512
 // consecutive tiles to the XCDs in turn.  Either order with one tile per
 // workgroup beat persistent grid-stride loops.

@@ -5,9 +5,9 @@
 // rules for how many workgroups of a large optimizer launch stay resident
 // per CU, with each order's own budgets (at the end).
 //
-// Two orders.  Large optimizer launches with much arithmetic per byte take
-// their tiles in sequence, workgroup b tile b (use_sequence below); every
-// other launch takes the chunked order that follows.
+// Two orders.  Large optimizer launches with BF16 parameters take their tiles
+// in sequence, workgroup b tile b (use_sequence below); every other launch
+// takes the chunked order that follows.
 //
 // Chunked order.  The dispatcher hands workgroup b to XCD (b mod 8).  Tiles are dealt to the
 // XCDs in chunks of 2^s consecutive tiles: XCD x takes chunks x, x + 8,
@@ -81,25 +81,19 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
 // chip is one window per stream, a few MiB wide; the chunked order has eight,
 // one an XCD.  HBM serves several streams the worse the wider the addresses in
 // flight spread, and the more of them there are (the caps below).  Launches
-// whose workgroups live long need many in flight, so there the narrower
-// window pays.  Their tile-map entries come from more cache lines, since
-// neighbouring tiles run on different XCDs, which is why launches of FP32
-// parameters and gradients with cheap or wide moments stay chunked: in
-// sequence they measured 0 to 2% less (BF16-SR moments, 1.55 * 10^9 elements:
-// 4.85 against 4.79 ms; FP32 moments, 7.4 * 10^8: 6.21 against 6.36 TB/s).
+// with BF16 parameters do much arithmetic per byte: their workgroups live long,
+// so many have to be in flight, and the narrower window pays.
 //
-// MI355X, 24 tensors, mean over 6 placements, TB/s, chunked at its own best
-// cap -> in sequence at its best, at 2.6 * 10^8 and 7.4 * 10^8 elements:
-// BF16 p/g with BF16-SR m/v 6.42 -> 6.53 and 6.29 -> 6.51, BF16-nearest 6.31
-// -> 6.59 and 6.23 -> 6.58, FP32 6.14 -> 6.47 and 6.10 -> 6.39, E4M3-SR m 6.12
-// -> 6.31 and 6.13 -> 6.26, FP16-SR 6.14 -> 6.33 and 6.14 -> 6.25; FP32 p with
-// BF16 g and BF16-SR m/v 6.39 -> 6.58 and 6.30 -> 6.56, FP8-nearest 6.44 -> 6.56
-// and 6.32 -> 6.54 (1.3 and 5 * 10^8), FP16-SR 6.40 -> 6.45 and 6.23 -> 6.39;
-// FP32 p/g with E4M3-SR m 6.45 -> 6.57 and 6.36 -> 6.50.  SGDM with BF16 p/g
-// and FP32 momentum 6.51 -> 6.62, E4M3-SR 6.53 -> 6.80, with BF16 g 6.58 -> 6.63.
-// Level or worse, hence chunked: FP32 p/g with two FP8-SR moments (-1.3 to
-// +0.5%) or two FP16-SR ones (-0.6 to +1%), SGDM with FP32 p/g (-0.9%), and
-// SGDM with BF16 p/g and BF16 momentum (10 B: -2.5 to 0%).
+// MI355X, through AdamW over 50 tensors, 1.55 * 10^9 elements, chunked (no cap
+// helps there) -> in sequence at its cap, ms: BF16-SR m/v 3.473 -> 3.314,
+// E4M3-SR m + BF16-SR v 2.951 -> 2.905, FP16-SR m/v 3.460 -> 3.406.  24 tensors,
+// 2.6 * 10^8 and 7.4 * 10^8 elements, TB/s: BF16-nearest 6.31 -> 6.59 and 6.23 ->
+// 6.58, FP32 6.14 -> 6.47 and 6.10 -> 6.39, E4M3-nearest 6.35 -> 6.56 and 6.35
+// -> 6.44.  SGDM: FP32 momentum 6.51 -> 6.62, E4M3-SR 6.53 -> 6.80; BF16
+// momentum (10 B per element) -2.5 to 0%, so such SGDM launches stay chunked.
+// So do FP32 parameters: over separate allocations the sequence lost 1.8% on
+// GPT-2's shapes with BF16 gradients and 2.3% on 1.55 * 10^9 elements with
+// E4M3-SR + BF16-SR moments, though over flat buffers it gained as much.
 //
 // From 5 * 2^21 elements on; below, the chunked order is level or better.
 constexpr uint64_t kSequenceMinElements = 5ull << 21;
@@ -107,12 +101,9 @@ constexpr uint64_t kSequenceMinElements = 5ull << 21;
 // `moments` is 2 for AdamW and 1 for SGDM, `minifloat_sr` counts the moments
 // that round stochastically to FP16 or FP8.
 SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params,
-                                        bool bf16_gradient, uint32_t moments, uint32_t minifloat_sr,
-                                        uint32_t bytes_per_element) {
-  const bool long_lived = bf16_params     ? moments == 2 || minifloat_sr > 0 || bytes_per_element >= 14
-                          : bf16_gradient ? bytes_per_element <= 18
-                                          : minifloat_sr == 1 && bytes_per_element >= 18 && bytes_per_element <= 20;
-  return long_lived && static_cast<uint64_t>(tiles) * block * lanes >= kSequenceMinElements;
+                                        uint32_t moments, uint32_t minifloat_sr, uint32_t bytes_per_element) {
+  return bf16_params && (moments == 2 || minifloat_sr > 0 || bytes_per_element >= 14) &&
+         static_cast<uint64_t>(tiles) * block * lanes >= kSequenceMinElements;
 }
 
 // Grid of a launch in sequence: `tiles` workgroups, in rows where one
@@ -197,14 +188,13 @@ SR_HOST_DEVICE inline uint32_t resident_cap(uint32_t tiles, uint32_t block, uint
 }
 
 // Bytes of tiles in flight per CU of a launch in sequence, where the rate
-// peaked on MI355X over 26 combinations of operand types (caps 5 to 14 and
-// none, as above): 88 KiB, 96 with one moment that rounds stochastically to
-// FP16 or FP8, 104 with two; a cap past kResidentCapMax means none, as in the
-// chunked order.  The caps this gives, best measured in parentheses: BF16 p/g
-// with BF16-SR m/v 13 (12-13, which reserve alike), BF16-nearest 13 (11-12),
-// FP32 8 (7-9), E4M3-SR m none (none), FP16-SR none (none); BF16 g with BF16-SR
-// 10 (9-10), FP8-nearest 13 (12), E4M3-SR m 12 (12-14), FP16-SR m 11 (10-11),
-// two FP16-SR 12 (11-12), two E4M3-SR none (none); FP32 p/g with E4M3-SR m 11 (10-11).
+// peaked on MI355X (caps 5 to 14 and none, as above): 88 KiB, 96 with one
+// moment that rounds stochastically to FP16 or FP8, 104 with two; a cap past
+// kResidentCapMax means none, as in the chunked order.  The caps this gives,
+// best measured in parentheses: AdamW with BF16-SR m/v 13 (12-13, which reserve
+// alike), BF16-nearest 13 (11-12), FP32 8 (7-9), E4M3-SR + BF16-SR none (none),
+// FP16-SR + BF16-SR 14 (14 or none), E5M2-SR + FP32 12 (11-12), two FP16-SR none
+// (none); SGDM with FP32 momentum 13 (12-14), E4M3-SR none (none).
 SR_HOST_DEVICE constexpr uint32_t sequence_in_flight(uint32_t minifloat_sr) {
   return (88u + 8u * minifloat_sr) * 1024u;
 }
