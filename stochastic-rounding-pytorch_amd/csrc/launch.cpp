@@ -61,6 +61,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/ops/empty_like.h>
 #include <c10/core/DeviceGuard.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
@@ -204,7 +205,10 @@ c10::ScalarType scalar_type(int code) {
   }
 }
 
+// Torch's own translation of its exceptions around the allocation: an
+// allocator that is out of memory raises torch.OutOfMemoryError.
 PyObject* cast_new(PyObject*, PyObject* args) {
+  HANDLE_TH_ERRORS
   PyObject* x_obj;
   int code, rule, threads;
   unsigned long long seed, offset, stream;
@@ -217,16 +221,24 @@ PyObject* cast_new(PyObject*, PyObject* args) {
   }
   if (g_cast == nullptr) return fail(PyExc_RuntimeError, "the native entries are not bound to the library");
   at::Tensor out;
-  int status = 0;
-  const bool ran = run_on_device(x.device(), [&] {
+  {
+    const pybind11::gil_scoped_release no_gil;
     out = at::empty_like(x, x.options().dtype(scalar_type(code)), at::MemoryFormat::Contiguous);
-    if (x.numel() == 0) return;
-    TORCH_CHECK_VALUE(x.const_data_ptr() != nullptr, "tensors without device memory cannot be cast");
-    status = g_cast(x.const_data_ptr(), out.data_ptr(), x.numel(), code, rule, static_cast<uint32_t>(seed),
-                    static_cast<uint32_t>(offset), threads, address(stream));
-  });
-  if (!ran) return nullptr;
+  }
+  const int64_t n = x.numel();
+  if (n == 0) return THPVariable_Wrap(std::move(out));
+  const void* source = x.const_data_ptr();
+  void* target = out.data_ptr();
+  if (!source || !target) return fail(PyExc_ValueError, "tensors without device memory cannot be cast");
+  int status = 0;
+  if (!run_on_device(x.device(), [&] {
+        status = g_cast(source, target, n, code, rule, static_cast<uint32_t>(seed), static_cast<uint32_t>(offset),
+                        threads, address(stream));
+      })) {
+    return nullptr;
+  }
   return status ? PyLong_FromLong(status) : THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
 }
 
 // The tensor checks of the fused updates, in the validating order of
@@ -398,7 +410,7 @@ PyObject* guarded(PyObject* self, PyObject* args) {
 
 PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, "Keep the addresses of the C ABI's entry points."},
-    {"cast_new", guarded<cast_new>, METH_VARARGS, "Cast into a new tensor; returns it, a nonzero status, or None."},
+    {"cast_new", cast_new, METH_VARARGS, "Cast into a new tensor; returns it, a nonzero status, or None."},
     {"adamw_multi", guarded<adamw_multi>, METH_VARARGS, "Call sr_adamw_multi on a device; returns its status."},
     {"sgdm_multi", guarded<sgdm_multi>, METH_VARARGS, "Call sr_sgdm_multi on a device; returns its status."},
     {"cast", guarded<cast>, METH_VARARGS, "Check the tensors and call sr_cast; returns its status."},

@@ -1,0 +1,90 @@
+"""``step()`` outside torch's profiler range unless something would see it.
+
+The range, and torch's global and per-optimizer step hooks, come from the
+wrapper torch puts around every optimizer's step; an unobserved step leaves
+it out.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+from torch.optim.optimizer import register_optimizer_step_post_hook, register_optimizer_step_pre_hook
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from sr_states import _group_walk
+from sr_states.optim._state import StateOptimizer
+
+
+class Counting(StateOptimizer):
+    _state_names = ("momentum_buffer",)
+
+    def __init__(self, params):
+        super().__init__(params, {"lr": 0.1})
+        self.updates = 0
+
+    def _step_group(self, group, formats, items, rng_step):
+        assert not torch.is_grad_enabled()
+        self.updates += 1
+
+
+class Overriding(Counting):
+    def step(self, closure=None):
+        return super().step(closure)
+
+
+def _optimizer(cls=Counting):
+    return cls([torch.nn.Parameter(torch.zeros(3))])
+
+
+def test_a_plain_step_runs_once_and_returns_the_closure_loss():
+    optimizer = _optimizer()
+    assert not optimizer._step_observed()
+    assert optimizer.step(lambda: torch.tensor(2.0, requires_grad=True) * 3) == 6.0
+    assert optimizer.updates == 1 and torch.is_grad_enabled()
+
+
+@pytest.mark.parametrize("cls", [Counting, Overriding])
+def test_step_hooks_run_once_and_may_replace_the_arguments(cls):
+    optimizer, seen = _optimizer(cls), []
+    handles = [
+        register_optimizer_step_pre_hook(lambda o, args, kwargs: seen.append("global pre")),
+        register_optimizer_step_post_hook(lambda o, args, kwargs: seen.append("global post")),
+        optimizer.register_step_pre_hook(lambda o, args, kwargs: ((o, lambda: 5.0), {})),
+        optimizer.register_step_post_hook(lambda o, args, kwargs: seen.append("post")),
+    ]
+    try:
+        assert optimizer.step() == 5.0
+    finally:
+        for handle in handles:
+            handle.remove()
+    assert sorted(seen) == ["global post", "global pre", "post"] and optimizer.updates == 1
+    optimizer.step()
+    assert len(seen) == 3 and optimizer.updates == 2
+
+
+def test_a_profiler_sees_the_step_range():
+    optimizer = _optimizer()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as profile:
+        assert _group_walk.observed()
+        optimizer.step()
+    assert any(event.key == "Optimizer.step#Counting.step" for event in profile.key_averages())
+    assert not _group_walk.observed()
+
+
+def test_a_dispatch_mode_counts_as_an_observer():
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert _group_walk.observed()
+    assert not _group_walk.observed()
+
+
+def test_a_scheduler_still_tracks_the_step():
+    optimizer = _optimizer()
+    scheduler = torch.optim.lr_scheduler.StepLR(optimizer, 1)
+    optimizer.step()
+    scheduler.step()
+    assert optimizer.updates == 1
