@@ -86,7 +86,8 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
 //
 // MI355X, through AdamW over 50 tensors, 1.55 * 10^9 elements, chunked (no cap
 // helps there) -> in sequence at its cap, ms: BF16-SR m/v 3.473 -> 3.314,
-// E4M3-SR m + BF16-SR v 2.951 -> 2.905, FP16-SR m/v 3.460 -> 3.406.  24 tensors,
+// E4M3-SR m + BF16-SR v 2.951 -> 2.905, FP16-SR m/v 3.460 -> 3.406 (on another
+// machine, in turn twice, 2.985 -> 2.979 and 3.510 -> 3.477).  24 tensors,
 // 2.6 * 10^8 and 7.4 * 10^8 elements, TB/s: BF16-nearest 6.31 -> 6.59 and 6.23 ->
 // 6.58, FP32 6.14 -> 6.47 and 6.10 -> 6.39, E4M3-nearest 6.35 -> 6.56 and 6.35
 // -> 6.44.  SGDM: FP32 momentum 6.51 -> 6.62, E4M3-SR 6.53 -> 6.80; BF16
