@@ -9,7 +9,7 @@
 // tried (E4M3 + BF16 moments 6.03 vs 5.41 TB/s at E = 8, BF16 parameters
 // and momentum 6.47 vs 6.21) and E = 8 the faster cast width (BF16 output
 // 6.08 vs 5.81 TB/s).  Rows of any alignment take the same accesses: a
-// group's alignment is declared as one element's (GroupAccess), which gfx950
+// group's alignment is declared as one element's (sr_group_access.h), which gfx950
 // serves with the same instructions.  Measured on MI355X against one access
 // per element for rows off 16-byte alignment, per launch: FP16-SR moments on
 // packed FP32 gradients, 230 M elements 882 -> 700 us, 49 M 177 -> 155;
@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/sr_states_hip.h"
+#include "sr_group_access.h"
 #include "sr_math.h"
 #include "sr_tile_order.h"
 
@@ -88,69 +89,9 @@ __device__ __forceinline__ uint32_t logical_tile(uint32_t total_tiles, bool in_s
 }
 
 // ---------------------------------------------------------------------------
-// Element I/O.  Raw storage words are zero-extended into 32-bit lanes.  Table
-// entries are plain integers, so pointers are cast to the global address
-// space explicitly; otherwise every access would be a flat access.
+// Element I/O.  Raw storage words are zero-extended into 32-bit lanes; the
+// accesses themselves are in sr_group_access.h.
 // ---------------------------------------------------------------------------
-#if defined(__HIP_DEVICE_COMPILE__)
-#define SR_GLOBAL __attribute__((address_space(1)))
-#else
-#define SR_GLOBAL
-#endif
-
-template <class T>
-__device__ __forceinline__ const SR_GLOBAL T* gptr(const void* p) {
-  return (const SR_GLOBAL T*)(p);
-}
-template <class T>
-__device__ __forceinline__ SR_GLOBAL T* gptr_mut(void* p) {
-  return (SR_GLOBAL T*)(p);
-}
-
-// Streaming accesses.  Every operand is read once and written at most once
-// per launch, so every global load and store carries the non-temporal hint.
-// Measured on MI355X: north star 5.64 -> 6.13 TB/s, SGDM 5.87 -> 6.41 TB/s;
-// the hint on loads alone is slower (5.51) and on stores alone neutral.
-template <class T>
-__device__ __forceinline__ T stream_load(const void* p) {
-  return __builtin_nontemporal_load(gptr<T>(p));
-}
-template <class T>
-__device__ __forceinline__ void stream_store(void* p, T v) {
-  __builtin_nontemporal_store(v, gptr_mut<T>(p));
-}
-
-// The words of one group of four elements, moved as one access.  The types
-// promise the alignment of one element only, so groups of views that start
-// anywhere move the same way: gfx950's global accesses take any alignment,
-// and an access that is aligned costs what a declared alignment would.
-template <int BYTES>
-struct GroupAccess;
-template <>
-struct GroupAccess<16> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4))); };
-template <>
-struct GroupAccess<8> { typedef uint32_t type __attribute__((ext_vector_type(2), aligned(2))); };
-template <>
-struct GroupAccess<4> { typedef uint32_t type __attribute__((aligned(1))); };
-
-// kCached keeps the load under the normal cache policy (the small casts'
-// input, below).
-template <int BYTES, bool kCached = false>
-__device__ __forceinline__ void load_words(const char* ptr, uint32_t* w) {
-  using T = typename GroupAccess<BYTES>::type;
-  T a;
-  if constexpr (kCached) a = *gptr<T>(ptr);
-  else a = stream_load<T>(ptr);
-  __builtin_memcpy(w, &a, BYTES);
-}
-
-template <int BYTES>
-__device__ __forceinline__ void store_words(char* ptr, const uint32_t* w) {
-  using T = typename GroupAccess<BYTES>::type;
-  T a;
-  __builtin_memcpy(&a, w, BYTES);
-  stream_store<T>(ptr, a);
-}
 
 // The storage words of the group of four elements at index i, moved as one
 // access.
