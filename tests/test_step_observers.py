@@ -88,3 +88,30 @@ def test_a_scheduler_still_tracks_the_step():
     optimizer.step()
     scheduler.step()
     assert optimizer.updates == 1
+
+
+@pytest.mark.parametrize("call,positional,named", [
+    (lambda o, f: o.step(), 0, ()),
+    (lambda o, f: o.step(None), 1, ()),
+    (lambda o, f: o.step(f), 1, ()),
+    (lambda o, f: o.step(closure=f), 0, ("closure",)),
+])
+def test_step_hooks_see_the_call_as_it_was_made(call, positional, named):
+    optimizer, seen = _optimizer(), []
+    optimizer.register_step_pre_hook(lambda o, args, kwargs: seen.append((args[0] is o, len(args), tuple(kwargs))))
+    optimizer.register_step_post_hook(lambda o, args, kwargs: seen.append((args[0] is o, len(args), tuple(kwargs))))
+    call(optimizer, lambda: 2.0)
+    assert seen == [(True, 1 + positional, named)] * 2 and optimizer.updates == 1
+
+
+def test_a_pre_hook_may_add_the_closure_by_name():
+    optimizer = _optimizer()
+    optimizer.register_step_pre_hook(lambda o, args, kwargs: (args, {**kwargs, "closure": lambda: 5.0}))
+    assert optimizer.step() == 5.0 and optimizer.updates == 1
+
+
+def test_a_subclass_may_use_the_name_of_an_inner_step():
+    optimizer = _optimizer()
+    optimizer._step = 0
+    optimizer.step()
+    assert optimizer.updates == 1 and optimizer._step == 0
