@@ -7,6 +7,8 @@ it out.
 
 from __future__ import annotations
 
+import functools
+
 import pytest
 import torch
 from torch.optim.optimizer import register_optimizer_step_post_hook, register_optimizer_step_pre_hook
@@ -115,3 +117,77 @@ def test_a_subclass_may_use_the_name_of_an_inner_step():
     optimizer._step = 0
     optimizer.step()
     assert optimizer.updates == 1 and optimizer._step == 0
+
+
+def _patched_after_construction(base):
+    class Patched(base):
+        pass
+
+    optimizer, inherited = _optimizer(Patched), Patched.step
+
+    @functools.wraps(inherited)
+    def step(self, *args, **kwargs):
+        return inherited(self, *args, **kwargs)
+
+    Patched.step = step
+    return optimizer
+
+
+def _patched_before_construction(base):
+    class Patched(base):
+        pass
+
+    @functools.wraps(Patched.step)
+    def step(self, *args, **kwargs):
+        return base.step(self, *args, **kwargs)
+
+    Patched.step = step
+    return _optimizer(Patched)
+
+
+def _override_named_like_the_inherited(base):
+    class Override(base):
+        @functools.wraps(base.step)
+        def step(self, closure=None):
+            return super().step(closure)
+
+    return _optimizer(Override)
+
+
+def _override_named_like_the_base(base):
+    class Override(base):
+        @functools.wraps(StateOptimizer.step)
+        def step(self, closure=None):
+            return super().step(closure)
+
+    return _optimizer(Override)
+
+
+@pytest.mark.parametrize("constructed", [False, True])
+@pytest.mark.parametrize("make", [_patched_after_construction, _patched_before_construction,
+                                  _override_named_like_the_inherited, _override_named_like_the_base])
+def test_patched_and_wrapped_steps_keep_hooks_and_range(make, constructed):
+    class Base(Counting):
+        pass
+
+    if constructed:  # torch has wrapped the base class's step, and marked it as wrapped
+        _optimizer(Base)
+    optimizer, seen = make(Base), []
+    optimizer.register_step_pre_hook(lambda *a: seen.append("pre"))
+    optimizer.register_step_post_hook(lambda *a: seen.append("post"))
+    optimizer.step()
+    assert seen == ["pre", "post"] and optimizer.updates == 1
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as profile:
+        optimizer.step()
+    assert sum(event.key.startswith("Optimizer.step#") for event in profile.key_averages()) == 1
+
+
+def test_a_step_within_a_step_has_hooks_of_its_own():
+    optimizer, seen = _optimizer(Overriding), []
+    optimizer.register_step_post_hook(lambda o, args, kwargs: seen.append(o.updates))
+    optimizer.step(lambda: optimizer.step())
+    assert seen == [1, 2]
+    with pytest.raises(ZeroDivisionError):
+        optimizer.step(lambda: 1 / 0)
+    optimizer.step()
+    assert seen == [1, 2, 3]
