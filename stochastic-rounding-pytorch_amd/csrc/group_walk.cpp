@@ -40,11 +40,12 @@
 //
 // observed() -> bool
 //   Whether anything in this process or thread would see a profiler range:
-//   a record-function callback (every profiler, of this thread or global)
-//   or a torch dispatch mode.
+//   a record-function callback (every profiler, of this thread or global),
+//   a torch dispatch mode or a torch function mode.
 
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/record_function.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <structmember.h>
@@ -406,7 +407,8 @@ PyObject* set_steps(PyObject*, PyObject* args) {
 }
 
 PyObject* observed(PyObject*, PyObject*) {
-  return PyBool_FromLong(at::hasCallbacks() || c10::impl::TorchDispatchModeTLS::any_modes_set());
+  return PyBool_FromLong(at::hasCallbacks() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+                         at::impl::torch_function_mode_enabled());
 }
 
 // enable_spec_fast_path(spec_type): compare DTensor gradient specs of this

@@ -12,6 +12,7 @@ import functools
 import pytest
 import torch
 from torch.optim.optimizer import register_optimizer_step_post_hook, register_optimizer_step_pre_hook
+from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from sr_states import _group_walk
@@ -191,3 +192,20 @@ def test_a_step_within_a_step_has_hooks_of_its_own():
         optimizer.step(lambda: 1 / 0)
     optimizer.step()
     assert seen == [1, 2, 3]
+
+
+def test_a_function_mode_sees_the_step_range():
+    class Mode(TorchFunctionMode):
+        def __init__(self):
+            self.seen = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.seen.append(func.__name__)
+            return func(*args, **(kwargs or {}))
+
+    optimizer = _optimizer()
+    with Mode() as mode:
+        assert _group_walk.observed()
+        optimizer.step()
+    assert "_record_function_enter_new" in mode.seen and optimizer.updates == 1
+    assert not _group_walk.observed()
