@@ -209,3 +209,32 @@ def test_a_function_mode_sees_the_step_range():
         optimizer.step()
     assert "_record_function_enter_new" in mode.seen and optimizer.updates == 1
     assert not _group_walk.observed()
+
+
+@pytest.mark.parametrize("scope", ["optimizer", "global"])
+def test_a_post_hook_registered_by_the_closure_runs_after_the_step(scope):
+    optimizer, seen, handles = _optimizer(), [], []
+
+    def hook(o, args, kwargs):
+        seen.append((o.updates, len(args), tuple(kwargs)))
+
+    def closure():
+        handles.append(optimizer.register_step_post_hook(hook) if scope == "optimizer"
+                       else register_optimizer_step_post_hook(hook))
+        return 3.0
+
+    try:
+        assert optimizer.step(closure=closure) == 3.0
+    finally:
+        handles[0].remove()
+    assert seen == [(1, 1, ("closure",))]
+
+
+def test_an_unobserved_step_ends_in_the_step_code_method():
+    class Traced(Counting):
+        def _optimizer_step_code(self):
+            self.updates += 10
+
+    optimizer = _optimizer(Traced)
+    optimizer.step()
+    assert optimizer.updates == 11
