@@ -8,6 +8,7 @@ it out.
 from __future__ import annotations
 
 import functools
+import warnings
 
 import pytest
 import torch
@@ -238,3 +239,20 @@ def test_an_unobserved_step_ends_in_the_step_code_method():
     optimizer = _optimizer(Traced)
     optimizer.step()
     assert optimizer.updates == 11
+
+
+def test_a_compiled_step_traces_torchs_wrapper():
+    class Logging(Counting):
+        def _step_group(self, group, formats, items, rng_step):
+            log.append(torch.is_grad_enabled())
+
+    log, optimizer = [], _optimizer(Logging)
+    torch._dynamo.reset()
+    compiled = torch.compile(optimizer.step, backend="eager")
+    with warnings.catch_warnings(record=True) as caught:
+        warnings.simplefilter("always")
+        compiled()
+        compiled()
+    torch._dynamo.reset()
+    assert log == [False, False]
+    assert not [w for w in caught if "_group_walk" in str(w.message)]
