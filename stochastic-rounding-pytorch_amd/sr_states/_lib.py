@@ -195,6 +195,10 @@ def on_device(device: torch.device):
     return torch.cuda.device(device)
 
 
+# torch's setter of the grad mode: a torch.no_grad() around a small launch
+# costs several times as much.
+set_grad_enabled = getattr(torch._C, "_set_grad_enabled", None) or torch.set_grad_enabled
+
 _is_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", None) or torch.cuda.is_current_stream_capturing
 
 

@@ -86,10 +86,16 @@ def hip_adamw_step_(
     ``seed`` is the update key and ``offset`` the flat index of the first
     element.
     """
-    codes = resolve_native_codes(_STATE_NAMES, (exp_avg, exp_avg_sq), formats, rounding, block_size)
-    _validate_hyperparameters(lr, (beta1, beta2), eps, weight_decay)
-    _launch_step(parameter, gradient, exp_avg, exp_avg_sq, codes,
-                 adamw_scalars(lr, beta1, beta2, eps, weight_decay, _positive_step(step)), seed, offset, block_size)
+    grad = torch.is_grad_enabled()
+    _lib.set_grad_enabled(False)  # hyperparameters may be tensors that require gradients
+    try:
+        codes = resolve_native_codes(_STATE_NAMES, (exp_avg, exp_avg_sq), formats, rounding, block_size)
+        _validate_hyperparameters(lr, (beta1, beta2), eps, weight_decay)
+        _launch_step(parameter, gradient, exp_avg, exp_avg_sq, codes,
+                     adamw_scalars(lr, beta1, beta2, eps, weight_decay, _positive_step(step)), seed, offset,
+                     block_size)
+    finally:
+        _lib.set_grad_enabled(grad)
 
 
 def adamw_step_any_hyperparameters_(

@@ -65,11 +65,17 @@ def hip_sgdm_step_(
     any built-in storage format.  ``seed`` is the update key and ``offset``
     the flat index of the first element.
     """
-    codes = resolve_native_codes(_STATE_NAMES, (momentum,), formats, rounding, block_size)
-    nonnegative("learning rate", lr)
-    if not 0 <= momentum_factor < 1:
-        raise ValueError(f"invalid momentum value: {momentum_factor}")
-    _launch_step(parameter, gradient, momentum, codes, sgdm_scalars(lr, momentum_factor), seed, offset, block_size)
+    grad = torch.is_grad_enabled()
+    _lib.set_grad_enabled(False)  # hyperparameters may be tensors that require gradients
+    try:
+        codes = resolve_native_codes(_STATE_NAMES, (momentum,), formats, rounding, block_size)
+        nonnegative("learning rate", lr)
+        if not 0 <= momentum_factor < 1:
+            raise ValueError(f"invalid momentum value: {momentum_factor}")
+        _launch_step(parameter, gradient, momentum, codes, sgdm_scalars(lr, momentum_factor), seed, offset,
+                     block_size)
+    finally:
+        _lib.set_grad_enabled(grad)
 
 
 def sgdm_step_any_hyperparameters_(parameter, gradient, momentum, *, lr, momentum_factor, seed=0, offset=0,

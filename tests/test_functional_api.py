@@ -147,3 +147,32 @@ def test_argument_errors_come_before_device_checks():
         functional.sgdm_step(*tensors[:3], lr=0.1, momentum_factor=0.9, rounding="sideways")
     with pytest.raises(TypeError, match="must be tensors"):
         functional.sgdm_step(tensors[0], [0.0] * 8, tensors[2], lr=0.1, momentum_factor=0.9)
+
+
+@pytest.mark.parametrize("kind", ["adamw", "sgd"])
+def test_hyperparameters_may_require_gradients(monkeypatch, kind):
+    """A learning rate that autograd tracks is only a number to the update, which runs without grad mode."""
+    import importlib
+    import warnings
+
+    module = importlib.import_module(f"sr_states.hip.{kind}")
+    seen = []
+
+    def launch(*args):  # converts the scalars as the native entry does
+        scalars = next(a for a in args if isinstance(a, tuple) and not isinstance(a[0], tuple))
+        seen.append((torch.is_grad_enabled(), [float(s) for s in scalars]))
+
+    monkeypatch.setattr(module, "_launch_step", launch)
+    p, g, m, v = torch.zeros(4), torch.zeros(4), torch.zeros(4).bfloat16(), torch.zeros(4).bfloat16()
+    for lr in (0.5, torch.tensor(0.5, dtype=torch.float64, requires_grad=True)):
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            if kind == "adamw":
+                sr_states.hip_adamw_step_(p, g, m, v, **{**ADAMW, "lr": lr})
+            else:
+                sr_states.hip_sgdm_step_(p, g, m, lr=lr, momentum_factor=0.9, seed=0)
+        assert torch.is_grad_enabled()
+        with torch.no_grad(), pytest.raises(ValueError):
+            sr_states.hip_sgdm_step_(p, g, m, lr=-1.0, momentum_factor=0.9, seed=0)
+        assert torch.is_grad_enabled()
+    assert seen[0] == seen[1] and not seen[0][0]
