@@ -110,39 +110,39 @@ int cap_override() {
 // Whether an encoding rounds stochastically to FP16 or FP8.
 bool minifloat_sr(int enc) { return enc == sr::ENC_F16_SR || enc == sr::ENC_E4M3_SR || enc == sr::ENC_E5M2_SR; }
 
-// Launches an optimizer kernel over a.total_tiles tiles of block * lanes
-// elements in the order its size and operands ask for, with that order's cap
-// on the resident workgroups.  `chunked_in_flight` is the chunked order's
-// budget, `moments_sr` how many of the `moments` are minifloat_sr.
-template <class Args>
-int launch_update(const void* fn, Args& a, int block, int lanes, bool bf16_params, uint32_t moments,
-                  uint32_t moments_sr, uint32_t bytes, uint32_t chunked_in_flight, void* stream) {
-  const uint32_t tiles = a.total_tiles, b = static_cast<uint32_t>(block), l = static_cast<uint32_t>(lanes);
-  a.in_sequence = sr::use_sequence(tiles, b, l, bf16_params, moments, moments_sr, bytes);
-  uint32_t cap;
-  if (cap_override() >= 0) {
-    cap = a.in_sequence || tiles >= sr::kResidentCapMinTiles ? static_cast<uint32_t>(cap_override()) : 0u;
-  } else if (a.in_sequence) {
-    cap = sr::workgroups_in(sr::sequence_in_flight(moments_sr), b, l, bytes);
-  } else {
-    cap = sr::resident_cap(tiles, b, l, bytes, !bf16_params, chunked_in_flight);
-  }
-  return launch(fn, block, tiles, &a, stream, a.in_sequence, cap);
+// Resident-workgroup cap of a launch in the chunked order (sr::resident_cap).
+uint32_t chunked_cap(uint32_t tiles, int block, int lanes, uint32_t bytes, bool fp32_params, uint32_t in_flight) {
+  if (cap_override() >= 0) return tiles >= sr::kResidentCapMinTiles ? static_cast<uint32_t>(cap_override()) : 0u;
+  return sr::resident_cap(tiles, static_cast<uint32_t>(block), static_cast<uint32_t>(lanes), bytes, fp32_params,
+                          in_flight);
 }
 
+// Launches an AdamW kernel over a.total_tiles tiles in the order its size and
+// operands ask for, with that order's cap on the resident workgroups.
 int launch_adamw(sr::AdamWArgs& a, int pi, int gi, int me, int ve, int block, void* stream) {
   const uint32_t bytes = 2 * sr::enc_bytes(param_enc(pi)) + sr::enc_bytes(param_enc(gi)) + 2 * sr::enc_bytes(me) +
                          2 * sr::enc_bytes(ve);
-  return launch_update(tables().adamw[pi][gi][me][ve], a, block,
-                       sr::lane_elements(param_enc(pi), param_enc(gi), me, ve), pi == 1, 2,
-                       static_cast<uint32_t>(minifloat_sr(me)) + minifloat_sr(ve), bytes,
-                       sr::adamw_in_flight(gi == 1, minifloat_sr(me) && minifloat_sr(ve)), stream);
+  const int lanes = sr::lane_elements(param_enc(pi), param_enc(gi), me, ve);
+  const uint32_t b = static_cast<uint32_t>(block), l = static_cast<uint32_t>(lanes);
+  a.in_sequence = sr::use_sequence(a.total_tiles, b, l, pi == 1);
+  uint32_t cap;
+  if (!a.in_sequence) {
+    cap = chunked_cap(a.total_tiles, block, lanes, bytes, pi == 0,
+                      sr::adamw_in_flight(gi == 1, minifloat_sr(me) && minifloat_sr(ve)));
+  } else if (cap_override() >= 0) {
+    cap = static_cast<uint32_t>(cap_override());
+  } else {
+    cap = sr::workgroups_in(sr::sequence_in_flight(static_cast<uint32_t>(minifloat_sr(me)) + minifloat_sr(ve)), b, l,
+                            bytes);
+  }
+  return launch(tables().adamw[pi][gi][me][ve], block, a.total_tiles, &a, stream, a.in_sequence, cap);
 }
 
 int launch_sgdm(sr::SgdmArgs& a, int pi, int gi, int ue, int block, void* stream) {
   const uint32_t bytes = 2 * sr::enc_bytes(param_enc(pi)) + sr::enc_bytes(param_enc(gi)) + 2 * sr::enc_bytes(ue);
-  return launch_update(tables().sgdm[pi][gi][ue], a, block, sr::lane_elements(param_enc(pi), param_enc(gi), ue, ue),
-                       pi == 1, 1, minifloat_sr(ue), bytes, sr::sgdm_in_flight(ue == sr::ENC_F16_SR), stream);
+  const int lanes = sr::lane_elements(param_enc(pi), param_enc(gi), ue, ue);
+  return launch(tables().sgdm[pi][gi][ue], block, a.total_tiles, &a, stream, false,
+                chunked_cap(a.total_tiles, block, lanes, bytes, pi == 0, sr::sgdm_in_flight(ue == sr::ENC_F16_SR)));
 }
 
 // Tiles of block * lanes elements covering n elements, or fail if they do

@@ -5,7 +5,7 @@
 // rules for how many workgroups of a large optimizer launch stay resident
 // per CU, with each order's own budgets (at the end).
 //
-// Two orders.  Large optimizer launches with BF16 parameters take their tiles
+// Two orders.  Large AdamW launches with BF16 parameters take their tiles
 // in sequence, workgroup b tile b (use_sequence below); every other launch
 // takes the chunked order that follows.
 //
@@ -80,8 +80,8 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
 // Sequential order.  With workgroup b on tile b, what is in flight on the
 // chip is one window per stream, a few MiB wide; the chunked order has eight,
 // one an XCD.  HBM serves several streams the worse the wider the addresses in
-// flight spread, and the more of them there are (the caps below).  Launches
-// with BF16 parameters do much arithmetic per byte: their workgroups live long,
+// flight spread, and the more of them there are (the caps below).  AdamW with
+// BF16 parameters does much arithmetic per byte: its workgroups live long,
 // so many have to be in flight, and the narrower window pays.
 //
 // MI355X, through AdamW over 50 tensors, 1.55 * 10^9 elements, chunked (no cap
@@ -90,21 +90,24 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
 // machine, in turn twice, 2.985 -> 2.979 and 3.510 -> 3.477).  24 tensors,
 // 2.6 * 10^8 and 7.4 * 10^8 elements, TB/s: BF16-nearest 6.31 -> 6.59 and 6.23 ->
 // 6.58, FP32 6.14 -> 6.47 and 6.10 -> 6.39, E4M3-nearest 6.35 -> 6.56 and 6.35
-// -> 6.44.  SGDM: FP32 momentum 6.51 -> 6.62, E4M3-SR 6.53 -> 6.80; BF16
-// momentum (10 B per element) -2.5 to 0%, so such SGDM launches stay chunked.
-// So do FP32 parameters: over separate allocations the sequence lost 1.8% on
-// GPT-2's shapes with BF16 gradients and 2.3% on 1.55 * 10^9 elements with
-// E4M3-SR + BF16-SR moments, though over flat buffers it gained as much.
+// -> 6.44.
+//
+// Momentum SGD stays chunked.  With BF16 parameters and gradients, 50 tensors,
+// chunked -> in sequence, us: E4M3-SR momentum 167.9 -> 164.5 at 1.34 * 10^8
+// elements but 561 -> 599 at 4.5 * 10^8, 754 -> 793 at 6 * 10^8 and 1956 -> 2036
+// at 1.55 * 10^9 (E5M2-SR and one tensor alike); FP16-SR 203.1 -> 198.7, 685 ->
+// 695, 914 -> 928 and 2378 -> 2384; FP32 286.5 -> 286.6, 986 -> 985, 1313 -> 1304
+// and 3410 -> 3365; BF16 level.  So do FP32 parameters: over separate allocations
+// the sequence lost 1.8% on GPT-2's shapes with BF16 gradients and 2.3% on 1.55 *
+// 10^9 elements with E4M3-SR + BF16-SR moments, though over flat buffers it
+// gained as much.
 //
 // From 5 * 2^21 elements on; below, the chunked order is level or better.
 constexpr uint64_t kSequenceMinElements = 5ull << 21;
 
-// `moments` is 2 for AdamW and 1 for SGDM, `minifloat_sr` counts the moments
-// that round stochastically to FP16 or FP8.
-SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params,
-                                        uint32_t moments, uint32_t minifloat_sr, uint32_t bytes_per_element) {
-  return bf16_params && (moments == 2 || minifloat_sr > 0 || bytes_per_element >= 14) &&
-         static_cast<uint64_t>(tiles) * block * lanes >= kSequenceMinElements;
+// Whether an AdamW launch takes its tiles in sequence.
+SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params) {
+  return bf16_params && static_cast<uint64_t>(tiles) * block * lanes >= kSequenceMinElements;
 }
 
 // Grid of a launch in sequence: `tiles` workgroups, in rows where one
@@ -195,7 +198,7 @@ SR_HOST_DEVICE inline uint32_t resident_cap(uint32_t tiles, uint32_t block, uint
 // best measured in parentheses: AdamW with BF16-SR m/v 13 (12-13, which reserve
 // alike), BF16-nearest 13 (11-12), FP32 8 (7-9), E4M3-SR + BF16-SR none (none),
 // FP16-SR + BF16-SR 14 (14 or none), E5M2-SR + FP32 12 (11-12), two FP16-SR none
-// (none); SGDM with FP32 momentum 13 (12-14), E4M3-SR none (none).
+// (none).
 SR_HOST_DEVICE constexpr uint32_t sequence_in_flight(uint32_t minifloat_sr) {
   return (88u + 8u * minifloat_sr) * 1024u;
 }

@@ -29,9 +29,8 @@ int main() {
   }
   for (uint32_t block : {128u, 256u, 512u, 1024u}) {
     const uint32_t edge = static_cast<uint32_t>(sr::kSequenceMinElements / (block * 4));
-    if (!sr::use_sequence(edge, block, 4, true, 2, 0, 14) ||
-        sr::use_sequence(edge - 1, block, 4, true, 2, 0, 14) ||
-        sr::use_sequence(edge, block, 4, false, 2, 0, 20)) {
+    if (!sr::use_sequence(edge, block, 4, true) || sr::use_sequence(edge - 1, block, 4, true) ||
+        sr::use_sequence(0x7FFFF000u, block, 4, false)) {
       std::printf("block %u: the rule's edge moved\n", block);
       ++failures;
     }
