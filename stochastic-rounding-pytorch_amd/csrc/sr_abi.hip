@@ -124,7 +124,7 @@ int launch_adamw(sr::AdamWArgs& a, int pi, int gi, int me, int ve, int block, vo
                          2 * sr::enc_bytes(ve);
   const int lanes = sr::lane_elements(param_enc(pi), param_enc(gi), me, ve);
   const uint32_t b = static_cast<uint32_t>(block), l = static_cast<uint32_t>(lanes);
-  a.in_sequence = sr::use_sequence(a.total_tiles, b, l, pi == 1);
+  a.in_sequence = sr::use_sequence(a.total_tiles, b, l, pi == 1, bytes);
   uint32_t cap;
   if (!a.in_sequence) {
     cap = chunked_cap(a.total_tiles, block, lanes, bytes, pi == 0,

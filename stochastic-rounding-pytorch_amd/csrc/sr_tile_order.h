@@ -102,12 +102,25 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
 // 10^9 elements with E4M3-SR + BF16-SR moments, though over flat buffers it
 // gained as much.
 //
-// From 5 * 2^21 elements on; below, the chunked order is level or better.
-constexpr uint64_t kSequenceMinElements = 5ull << 21;
+// From how many elements on (of the tiles, partial ones counted whole).  Up to
+// 12 bytes per element (an FP8 moment in it): 5 * 2^21, where E4M3-SR + BF16-SR
+// goes 23.6 -> 23.4 us in one tensor and 23.9 -> 23.7 in twelve, E4M3-nearest
+// 19.6 -> 19.3 and 19.9 -> 19.2; at 2 * 10^7, 42.6 -> 41.6 and 34.6 -> 33.4.
+// Wider launches: 2^25.  Below that they are slower or level (us, one tensor;
+// twelve alike): at 10.5 * 10^6 BF16-SR 25.8 -> 26.1, FP32 37.9 -> 39.0, FP32
+// gradients 28.5 -> 29.3; at 2.5 * 10^7 55.6 -> 57.4, 86.4 -> 86.6 and (twelve)
+// 62.3 -> 64.1.  At 3.3 * 10^7, one tensor and fifty: BF16-SR 74.6 -> 73.6 and 75.8
+// -> 73.9, BF16-nearest 75.6 -> 72.1 and 73.0 -> 71.7, the others within 0.4%.
+constexpr uint64_t kSequenceMinElements = 1ull << 25;
+constexpr uint64_t kSequenceMinElementsNarrow = 5ull << 21;
+constexpr uint32_t kSequenceNarrowBytes = 12;
 
 // Whether an AdamW launch takes its tiles in sequence.
-SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params) {
-  return bf16_params && static_cast<uint64_t>(tiles) * block * lanes >= kSequenceMinElements;
+SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params,
+                                        uint32_t bytes_per_element) {
+  return bf16_params &&
+         static_cast<uint64_t>(tiles) * block * lanes >=
+             (bytes_per_element <= kSequenceNarrowBytes ? kSequenceMinElementsNarrow : kSequenceMinElements);
 }
 
 // Grid of a launch in sequence: `tiles` workgroups, in rows where one

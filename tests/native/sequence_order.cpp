@@ -27,12 +27,15 @@ int main() {
       }
     }
   }
+  // The least elements by the bytes per element, each side of the edge.
   for (uint32_t block : {128u, 256u, 512u, 1024u}) {
-    const uint32_t edge = static_cast<uint32_t>(sr::kSequenceMinElements / (block * 4));
-    if (!sr::use_sequence(edge, block, 4, true) || sr::use_sequence(edge - 1, block, 4, true) ||
-        sr::use_sequence(0x7FFFF000u, block, 4, false)) {
-      std::printf("block %u: the rule's edge moved\n", block);
-      ++failures;
+    for (uint32_t bytes : {10u, 12u, 13u, 14u, 16u, 22u}) {
+      const uint32_t edge = (bytes <= 12 ? 5u << 21 : 1u << 25) / (block * 4);
+      if (!sr::use_sequence(edge, block, 4, true, bytes) || sr::use_sequence(edge - 1, block, 4, true, bytes) ||
+          sr::use_sequence(0x7FFFF000u, block, 4, false, bytes)) {
+        std::printf("block %u, %u bytes: the rule's edge moved\n", block, bytes);
+        ++failures;
+      }
     }
   }
   for (uint32_t bytes = 6; bytes <= 28; ++bytes) {

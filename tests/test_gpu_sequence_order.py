@@ -1,10 +1,11 @@
 """Launches on both sides of the tile-order rule against the C oracle, byte for byte.
 
-From 5 * 2^21 elements on, launches with BF16 parameters take their tiles in
-sequence with a cap on the resident workgroups; one tile fewer, the chunked
-order.  The element count ends in a partial tile with a remainder, and the
-group spreads it over three tensors, one of which starts off 16-byte
-alignment.
+AdamW launches with BF16 parameters take their tiles in sequence, with a cap
+on the resident workgroups, from 5 * 2^21 elements on (up to 12 bytes per
+element) or from 2^25 on (more); one tile fewer, in the chunked order.  The
+rule counts whole tiles, so the sizes are chosen by tiles for each workgroup
+size.  The group spreads them over three tensors, each with a partial last
+tile and a remainder; the gradients start off 16-byte alignment.
 """
 
 from __future__ import annotations
@@ -16,18 +17,23 @@ from oracle import c_oracle, sr_oracle
 
 pytestmark = pytest.mark.gpu
 
-EDGE = 5 << 21
 BF16, F16, E4M3 = torch.bfloat16, torch.float16, torch.float8_e4m3fn
 
 
 @pytest.mark.parametrize("block_size", (128, 512))
-@pytest.mark.parametrize("total", (EDGE - 4 * 512 - 1, EDGE + 3))
-@pytest.mark.parametrize("moments", [(BF16, BF16), (F16, E4M3)])
-def test_both_sides_of_the_order_rule_equal_the_oracle(cuda, moments, total, block_size):
+@pytest.mark.parametrize("in_sequence", (False, True))
+@pytest.mark.parametrize("moments,edge", [((BF16, BF16), 1 << 25), ((F16, E4M3), 5 << 21)])
+def test_both_sides_of_the_order_rule_equal_the_oracle(cuda, moments, edge, in_sequence, block_size):
     import sr_states
 
     formats = tuple((dtype, "stochastic") for dtype in moments)
-    sizes = (1021, 4 * 1024 * 1024 + 1, total - 1021 - 4 * 1024 * 1024 - 1)
+    tile = 4 * block_size
+    sizes = [1021, 4 * 1024 * 1024 + 1]
+    tiles = edge // tile - (not in_sequence) - sum(-(-n // tile) for n in sizes)
+    sizes.append((tiles - 1) * tile + 3)
+    covered = sum(-(-n // tile) for n in sizes) * tile
+    assert (covered >= edge) == in_sequence and edge - tile <= covered <= edge
+    total = sum(sizes)
     generator = torch.Generator().manual_seed(total)
     params, grads = [], []
     for n in sizes:
