@@ -132,8 +132,7 @@ int launch_adamw(sr::AdamWArgs& a, int pi, int gi, int me, int ve, int block, vo
   } else if (cap_override() >= 0) {
     cap = static_cast<uint32_t>(cap_override());
   } else {
-    cap = sr::workgroups_in(sr::sequence_in_flight(static_cast<uint32_t>(minifloat_sr(me)) + minifloat_sr(ve)), b, l,
-                            bytes);
+    cap = sr::sequence_cap(static_cast<uint32_t>(minifloat_sr(me)) + minifloat_sr(ve), b, l, bytes);
   }
   return launch(tables().adamw[pi][gi][me][ve], block, a.total_tiles, &a, stream, a.in_sequence, cap);
 }

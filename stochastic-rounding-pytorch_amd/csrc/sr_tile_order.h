@@ -206,14 +206,25 @@ SR_HOST_DEVICE inline uint32_t resident_cap(uint32_t tiles, uint32_t block, uint
 
 // Bytes of tiles in flight per CU of a launch in sequence, where the rate
 // peaked on MI355X (caps 5 to 14 and none, as above): 88 KiB, 96 with one
-// moment that rounds stochastically to FP16 or FP8, 104 with two; a cap past
-// kResidentCapMax means none, as in the chunked order.  The caps this gives,
-// best measured in parentheses: AdamW with BF16-SR m/v 13 (12-13, which reserve
-// alike), BF16-nearest 13 (11-12), FP32 8 (7-9), E4M3-SR + BF16-SR none (none),
-// FP16-SR + BF16-SR 14 (14 or none), E5M2-SR + FP32 12 (11-12), two FP16-SR none
-// (none).
+// moment that rounds stochastically to FP16 or FP8, 104 with two.
 SR_HOST_DEVICE constexpr uint32_t sequence_in_flight(uint32_t minifloat_sr) {
   return (88u + 8u * minifloat_sr) * 1024u;
+}
+
+// The cap of a launch in sequence: what that budget gives, and none where it
+// gives more than 13 workgroups of 128 lanes.  The caps this gives, best
+// measured in parentheses: BF16-SR m/v 13 (12-13, which reserve alike),
+// BF16-nearest 13 (11-12), FP32 8 (7-9), E4M3-SR + BF16-SR none (none), FP16-SR +
+// BF16-SR none (none; 2.7 * 10^8 elements take 579 us with none, 596 at 14, 618
+// at 13), E5M2-SR + FP32 12 (12-13), FP16-SR + FP32 11 (11), two FP16-SR none (none).
+constexpr uint32_t kSequenceCapMax = 13;
+
+SR_HOST_DEVICE inline uint32_t sequence_cap(uint32_t minifloat_sr, uint32_t block, uint32_t lanes,
+                                            uint32_t bytes_per_element) {
+  const uint32_t in_flight = sequence_in_flight(minifloat_sr);
+  const uint32_t at_128 = workgroups_in(in_flight, 128, lanes, bytes_per_element);
+  if (at_128 == 0 || at_128 > kSequenceCapMax) return 0;
+  return workgroups_in(in_flight, block, lanes, bytes_per_element);
 }
 
 // The environment can replace the rule: SR_STATES_RESIDENT_CAP=k caps every

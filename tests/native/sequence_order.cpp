@@ -50,6 +50,19 @@ int main() {
       }
     }
   }
+  // The caps of 128-lane launches (none: 0), by moments that round
+  // stochastically to FP16 or FP8 and bytes per element; larger workgroups
+  // hold the same bytes, and none where 128 lanes would hold too many.
+  const uint32_t caps[][3] = {{0, 14, 13}, {0, 22, 8}, {0, 12, 0}, {0, 10, 0}, {1, 12, 0},
+                              {1, 14, 0},  {1, 16, 12}, {1, 18, 11}, {2, 14, 0}, {2, 16, 13}};
+  for (const auto& c : caps) {
+    const uint32_t wide = sr::sequence_cap(c[0], 512, 4, c[1]);
+    if (sr::sequence_cap(c[0], 128, 4, c[1]) != c[2] || (c[2] == 0) != (wide == 0) || 4 * wide > c[2] + 2) {
+      std::printf("%u moments, %u bytes: cap %u, %u at 512 lanes\n", c[0], c[1],
+                  sr::sequence_cap(c[0], 128, 4, c[1]), wide);
+      ++failures;
+    }
+  }
   std::printf("%d shapes, %d failures\n", shapes, failures);
   return failures != 0;
 }
