@@ -3,11 +3,11 @@
 // A kernel with trivial arithmetic (XORs) that moves exactly the streams of
 // one fused-update launch: a parameter (FP32 or BF16) read and written, a
 // gradient read, and one or two states read and written, with the product's
-// tile shape (128 lanes x 4 elements), its XCD-chunked tile order
-// (sr_tile_order.h), its addressing (a scalar tile base plus a 32-bit lane
-// offset), its non-temporal accesses and its resident-workgroup cap
-// (sr::resident_cap, enforced with sr::cap_lds as the library's launches
-// do).  Whatever rate this kernel reaches for n elements is what the memory
+// tile shape (128 lanes x 4 elements), its tile orders (sr_tile_order.h: in
+// chunks, and in sequence where the library takes that), its addressing (a
+// scalar tile base plus a 32-bit lane offset), its non-temporal accesses and
+// its resident-workgroup caps (sr::resident_cap and sr::sequence_cap, enforced
+// with sr::cap_lds as the library's launches do).  Whatever rate this kernel reaches for n elements is what the memory
 // system gives that access pattern at that footprint; the fused kernels do
 // strictly more work per byte, so their rate over this one says how much of
 // the reachable bandwidth their arithmetic and table lookups cost.
@@ -72,8 +72,10 @@ __device__ __forceinline__ void store(char* tile, uint32_t offset, typename Acce
 // states (V = 0: one state).  Tile t covers elements [t * kTile, (t + 1) *
 // kTile) < n.
 template <int P, int G, int M, int V>
-__global__ __launch_bounds__(kBlock) void streams(void* p, const void* g, void* m, void* v, uint32_t tiles) {
-  const uint32_t t = sr::tile_of(blockIdx.y * gridDim.x + blockIdx.x, tiles);
+__global__ __launch_bounds__(kBlock) void streams(void* p, const void* g, void* m, void* v, uint32_t tiles,
+                                                  uint32_t in_sequence) {
+  const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
+  const uint32_t t = in_sequence ? b : sr::tile_of(b, tiles);
   if (t >= tiles) return;
   const uint64_t first = static_cast<uint64_t>(t) * kTile;
   const uint32_t lane = threadIdx.x * kLanes;
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(kCastBlock) void cast_streams(const void* x, void* 
   }
 }
 
-typedef void (*Kernel)(void*, const void*, void*, void*, uint32_t);
+typedef void (*Kernel)(void*, const void*, void*, void*, uint32_t, uint32_t);
 
 Kernel pick(int p, int g, int m, int v) {
   if (p == 4) {
@@ -153,11 +155,11 @@ constexpr uint64_t kMaxGap = 16ull << 20;
 
 // Times the trivial kernel for one placement: streams p, g, m, v (widths
 // w[0..3], w[3] = 0 for one state) laid out from `slab` with `gap` bytes
-// after each (every base a multiple of 256 bytes).  Returns the milliseconds
-// per launch over `reps` launches after two untimed ones, or a negative
-// value on a HIP error.
+// after each (every base a multiple of 256 bytes), in the given tile order.
+// Returns the milliseconds per launch over `reps` launches after two untimed
+// ones, or a negative value on a HIP error.
 float time_placement(Kernel kernel, char* slab, const uint64_t (&bytes)[4], uint64_t gap, uint32_t tiles, int reps,
-                     size_t lds, hipEvent_t start, hipEvent_t stop) {
+                     uint32_t in_sequence, size_t lds, hipEvent_t start, hipEvent_t stop) {
   void* bases[4] = {nullptr, nullptr, nullptr, nullptr};
   uint64_t at = 0;
   for (int k = 0; k < 4; ++k) {
@@ -165,10 +167,10 @@ float time_placement(Kernel kernel, char* slab, const uint64_t (&bytes)[4], uint
     bases[k] = slab + at;
     at += (bytes[k] + 255) / 256 * 256 + gap;
   }
-  const sr::LaunchShape shape = sr::launch_shape(tiles, kBlock);
+  const sr::LaunchShape shape = in_sequence ? sr::sequence_shape(tiles, kBlock) : sr::launch_shape(tiles, kBlock);
   auto launch = [&] {
     hipLaunchKernelGGL(kernel, dim3(shape.x, shape.y), dim3(kBlock), lds, nullptr, bases[0], bases[1], bases[2],
-                       bases[3], tiles);
+                       bases[3], tiles, in_sequence);
   };
   launch();
   launch();
@@ -181,12 +183,17 @@ float time_placement(Kernel kernel, char* slab, const uint64_t (&bytes)[4], uint
   return ms / reps;
 }
 
+// A launch policy: the tile order and the resident-workgroup cap (0: none).
+struct Policy {
+  uint32_t in_sequence, cap;
+};
+
 // Times `kernel` over n elements at each gap in gaps[0..count) (every gap at
-// most kMaxGap) and each resident-workgroup cap in caps[0..ncaps) (0: none),
-// writing milliseconds per launch to ms[cap_index * count + gap_index].
-// Returns 0, or 2 for a HIP error (buffers are freed either way).
+// most kMaxGap) and each of `policies`, writing milliseconds per launch to
+// ms[policy_index * count + gap_index].  Returns 0, or 2 for a HIP error
+// (buffers are freed either way).
 int time_placements(Kernel kernel, uint64_t n, const int (&widths)[4], const uint64_t* gaps, int count,
-                    const uint32_t* caps, int ncaps, int reps, float* ms) {
+                    const Policy* policies, int npolicies, int reps, float* ms) {
   const uint32_t tiles = static_cast<uint32_t>(n / kTile);
   const uint64_t bytes[4] = {n * widths[0], n * widths[1], n * widths[2], n * widths[3]};
   uint64_t total = 0;
@@ -201,11 +208,11 @@ int time_placements(Kernel kernel, uint64_t n, const int (&widths)[4], const uin
       break;
     if (hipEventCreate(&start) != hipSuccess || hipEventCreate(&stop) != hipSuccess) break;
     bool failed = false;
-    for (int c = 0; c < ncaps && !failed; ++c) {
-      const size_t lds = sr::cap_lds(reinterpret_cast<const void*>(kernel), kBlock, caps[c]);
+    for (int c = 0; c < npolicies && !failed; ++c) {
+      const size_t lds = sr::cap_lds(reinterpret_cast<const void*>(kernel), kBlock, policies[c].cap);
       for (int i = 0; i < count && !failed; ++i) {
         float& out = ms[c * count + i];
-        out = time_placement(kernel, slab, bytes, gaps[i], tiles, reps, lds, start, stop);
+        out = time_placement(kernel, slab, bytes, gaps[i], tiles, reps, policies[c].in_sequence, lds, start, stop);
         failed = out < 0.0f;
       }
     }
@@ -236,35 +243,54 @@ __global__ void fill_update_inputs(float* p, float* g, uint64_t n) {
 // Average milliseconds per launch of the trivial kernel over n elements with
 // a parameter of p_bytes, a gradient of g_bytes and states of m_bytes and
 // v_bytes per element (v_bytes 0: one state), over `reps` launches after two
-// untimed ones, at the best of the placements kCeilingGaps and of three
-// launch policies: no resident-workgroup cap, the cap of an 80 KiB budget
-// for this pattern (sr::resident_cap, the library's for FP32 gradients) and
-// half of it.  (With no arithmetic to wait
-// for, the trivial kernel's workgroups are short-lived and it keeps enough
-// bytes in flight with fewer of them: the north star's streams at 31 GB ran
-// at 6.18 TB/s uncapped, 6.31 at 8 per CU and 6.38 at 4.)  Supported
+// untimed ones, at the best of the placements kCeilingGaps and of several
+// launch policies: in chunks with no resident-workgroup cap, with the cap of
+// an 80 KiB budget for this pattern (sr::resident_cap, the library's for FP32
+// parameters and gradients) and with half of it; and where the library takes
+// this pattern in sequence (sr::use_sequence), in sequence with no cap, with
+// the library's caps for it (sr::sequence_cap) and with half of their budget.
+// (With no arithmetic to wait for, the trivial kernel's workgroups are
+// short-lived and it keeps enough bytes in flight with fewer of them: the
+// north star's streams at 31 GB ran at 6.18 TB/s uncapped, 6.31 at 8 per CU
+// and 6.38 at 4.)  Supported
 // (p, g, m, v) patterns: FP32 parameters with (4,2,2), (2,2,2), (4,1,2),
 // (4,2,0), (4,4,4), (4,1,1), (4,4,0), (4,1,0); BF16 parameters with (2,2,2),
 // (2,1,2), (2,2,0).  n must be a positive multiple of 512 with n / 512 <=
-// 2^31 - 4096 (the fused launches' tile limit); the grid is laid out as the
-// fused launches lay it out (sr::launch_shape).  Returns 0, or 1 for an
-// unsupported argument, 2 for a HIP error (buffers are freed either way).
+// 2^31 - 4096 (the fused launches' tile limit); each order's grid is laid out
+// as the fused launches lay it out (sr::launch_shape, sr::sequence_shape).
+// Returns 0, or 1 for an unsupported argument, 2 for a HIP error (buffers are
+// freed either way).
 extern "C" int sr_stream_ceiling_p(uint64_t n, int p_bytes, int g_bytes, int m_bytes, int v_bytes, int reps,
                                    float* avg_ms) {
   const Kernel kernel = pick(p_bytes, g_bytes, m_bytes, v_bytes);
   if (!kernel || !valid_streams(n, reps) || !avg_ms) return 1;
   const uint32_t per_element = 2 * p_bytes + g_bytes + 2 * m_bytes + 2 * v_bytes;
-  const uint32_t rule =
-      sr::resident_cap(static_cast<uint32_t>(n / kTile), kBlock, kLanes, per_element, p_bytes == 4);
-  uint32_t caps[3] = {0, rule, rule / 2};
-  const int ncaps = rule == 0 ? 1 : (rule / 2 == 0 ? 2 : 3);
+  const uint32_t tiles = static_cast<uint32_t>(n / kTile);
+  Policy policies[8];
+  int npolicies = 0;
+  auto add = [&](uint32_t in_sequence, uint32_t cap) {
+    for (int i = 0; i < npolicies; ++i)
+      if (policies[i].in_sequence == in_sequence && policies[i].cap == cap) return;
+    policies[npolicies++] = {in_sequence, cap};
+  };
+  const uint32_t rule = sr::resident_cap(tiles, kBlock, kLanes, per_element, p_bytes == 4);
+  add(0, 0);
+  add(0, rule);
+  add(0, rule / 2);
+  if (v_bytes && sr::use_sequence(tiles, kBlock, kLanes, p_bytes == 2, per_element)) {
+    // The formats of the states are open: none, one or two may round to FP16
+    // or FP8 stochastically.
+    add(1, 0);
+    for (uint32_t moments : {2u, 1u, 0u}) add(1, sr::sequence_cap(moments, kBlock, kLanes, per_element));
+    add(1, sr::workgroups_in(sr::sequence_in_flight(0) / 2, kBlock, kLanes, per_element));
+  }
   constexpr int kCount = sizeof(kCeilingGaps) / sizeof(kCeilingGaps[0]);
-  float ms[3 * kCount];
-  const int rc = time_placements(kernel, n, {p_bytes, g_bytes, m_bytes, v_bytes}, kCeilingGaps, kCount, caps, ncaps,
-                                 reps, ms);
+  float ms[8 * kCount];
+  const int rc = time_placements(kernel, n, {p_bytes, g_bytes, m_bytes, v_bytes}, kCeilingGaps, kCount, policies,
+                                 npolicies, reps, ms);
   if (rc != 0) return rc;
   float best = ms[0];
-  for (int i = 0; i < ncaps * kCount; ++i) best = ms[i] < best ? ms[i] : best;
+  for (int i = 0; i < npolicies * kCount; ++i) best = ms[i] < best ? ms[i] : best;
   *avg_ms = best;
   return 0;
 }
@@ -384,7 +410,7 @@ extern "C" int sr_launch_cap_sweep(uint64_t n, int reps, const int* caps, int nc
         }
         auto launch = [&] {
           if (kind) hipLaunchKernelGGL(fused, dim3(shape.x, shape.y), dim3(kBlock), lds, nullptr, a);
-          else hipLaunchKernelGGL(trivial, dim3(shape.x, shape.y), dim3(kBlock), lds, nullptr, p, g, m, v, tiles);
+          else hipLaunchKernelGGL(trivial, dim3(shape.x, shape.y), dim3(kBlock), lds, nullptr, p, g, m, v, tiles, 0u);
         };
         launch();
         launch();
