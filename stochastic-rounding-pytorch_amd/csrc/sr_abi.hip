@@ -124,15 +124,16 @@ int launch_adamw(sr::AdamWArgs& a, int pi, int gi, int me, int ve, int block, vo
                          2 * sr::enc_bytes(ve);
   const int lanes = sr::lane_elements(param_enc(pi), param_enc(gi), me, ve);
   const uint32_t b = static_cast<uint32_t>(block), l = static_cast<uint32_t>(lanes);
-  a.in_sequence = sr::use_sequence(a.total_tiles, b, l, pi == 1, bytes);
+  const uint32_t moments_sr = static_cast<uint32_t>(minifloat_sr(me)) + minifloat_sr(ve);
+  a.in_sequence = sr::use_sequence(a.total_tiles, b, l, pi == 1, moments_sr, bytes);
   uint32_t cap;
   if (!a.in_sequence) {
     cap = chunked_cap(a.total_tiles, block, lanes, bytes, pi == 0,
-                      sr::adamw_in_flight(gi == 1, minifloat_sr(me) && minifloat_sr(ve)));
+                      sr::adamw_in_flight(gi == 1, moments_sr == 2));
   } else if (cap_override() >= 0) {
     cap = static_cast<uint32_t>(cap_override());
   } else {
-    cap = sr::sequence_cap(static_cast<uint32_t>(minifloat_sr(me)) + minifloat_sr(ve), b, l, bytes);
+    cap = sr::sequence_cap(moments_sr, b, l, bytes);
   }
   return launch(tables().adamw[pi][gi][me][ve], block, a.total_tiles, &a, stream, a.in_sequence, cap);
 }

@@ -86,8 +86,9 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
 //
 // MI355X, through AdamW over 50 tensors, 1.55 * 10^9 elements, chunked (no cap
 // helps there) -> in sequence at its cap, ms: BF16-SR m/v 3.473 -> 3.314,
-// E4M3-SR m + BF16-SR v 2.951 -> 2.905, FP16-SR m/v 3.460 -> 3.406 (on another
-// machine, in turn twice, 2.985 -> 2.979 and 3.510 -> 3.477).  24 tensors,
+// E4M3-SR m + BF16-SR v 2.951 -> 2.905, FP16-SR m/v 3.460 -> 3.406; on other
+// machines 3.432 -> 3.338, 3.046 -> 2.982 (and 2.985 -> 2.979) and 3.554 -> 3.499
+// (and 3.510 -> 3.477).  24 tensors,
 // 2.6 * 10^8 and 7.4 * 10^8 elements, TB/s: BF16-nearest 6.31 -> 6.59 and 6.23 ->
 // 6.58, FP32 6.14 -> 6.47 and 6.10 -> 6.39, E4M3-nearest 6.35 -> 6.56 and 6.35
 // -> 6.44.
@@ -101,27 +102,6 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
 // the sequence lost 1.8% on GPT-2's shapes with BF16 gradients and 2.3% on 1.55 *
 // 10^9 elements with E4M3-SR + BF16-SR moments, though over flat buffers it
 // gained as much.
-//
-// From how many elements on (of the tiles, partial ones counted whole).  Up to
-// 12 bytes per element (an FP8 moment in it): 5 * 2^21, where E4M3-SR + BF16-SR
-// goes 23.6 -> 23.4 us in one tensor and 23.9 -> 23.7 in twelve, E4M3-nearest
-// 19.6 -> 19.3 and 19.9 -> 19.2; at 2 * 10^7, 42.6 -> 41.6 and 34.6 -> 33.4.
-// Wider launches: 2^25.  Below that they are slower or level (us, one tensor;
-// twelve alike): at 10.5 * 10^6 BF16-SR 25.8 -> 26.1, FP32 37.9 -> 39.0, FP32
-// gradients 28.5 -> 29.3; at 2.5 * 10^7 55.6 -> 57.4, 86.4 -> 86.6 and (twelve)
-// 62.3 -> 64.1.  At 3.3 * 10^7, one tensor and fifty: BF16-SR 74.6 -> 73.6 and 75.8
-// -> 73.9, BF16-nearest 75.6 -> 72.1 and 73.0 -> 71.7, the others within 0.4%.
-constexpr uint64_t kSequenceMinElements = 1ull << 25;
-constexpr uint64_t kSequenceMinElementsNarrow = 5ull << 21;
-constexpr uint32_t kSequenceNarrowBytes = 12;
-
-// Whether an AdamW launch takes its tiles in sequence.
-SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params,
-                                        uint32_t bytes_per_element) {
-  return bf16_params &&
-         static_cast<uint64_t>(tiles) * block * lanes >=
-             (bytes_per_element <= kSequenceNarrowBytes ? kSequenceMinElementsNarrow : kSequenceMinElements);
-}
 
 // Grid of a launch in sequence: `tiles` workgroups, in rows where one
 // dimension cannot hold them (launch_shape); workgroups past the last tile
@@ -225,6 +205,30 @@ SR_HOST_DEVICE inline uint32_t sequence_cap(uint32_t minifloat_sr, uint32_t bloc
   const uint32_t at_128 = workgroups_in(in_flight, 128, lanes, bytes_per_element);
   if (at_128 == 0 || at_128 > kSequenceCapMax) return 0;
   return workgroups_in(in_flight, block, lanes, bytes_per_element);
+}
+
+// Whether an AdamW launch takes its tiles in sequence: from how many elements
+// on (of the tiles, partial ones counted whole).  Launches without a cap, whose
+// arithmetic wants every workgroup: 5 * 2^21.  Two machines, chunked -> in
+// sequence, us, one tensor: E4M3-SR + BF16-SR 23.4 -> 23.2 at 1.05 * 10^7 elements
+// and 41.9 -> 41.0 at 2 * 10^7, E4M3-nearest 19.5 -> 19.2 and 34.2 -> 33.1, two
+// FP16-SR 27.0 -> 27.0 and 48.9 -> 47.5 (72.9 -> 69.7 at 3 * 10^7).
+// Launches with a cap: 2^25.  Below, it depends on the size, by how full the
+// last round of chunks is: BF16-SR 25.8 -> 26.1 at 1.05 * 10^7, 31.6 -> 31.2 at
+// 1.3 * 10^7, 55.6 -> 57.4 at 2.5 * 10^7, 66.9 -> 66.6 at 3 * 10^7; FP32 37.9 ->
+// 39.0, 46.7 -> 46.9, 86.4 -> 86.6, 104.4 -> 102.1; with FP32 gradients 28.5 ->
+// 29.3, 35.1 -> 35.3, 63.6 -> 63.6, 75.8 -> 75.5.  From there it mostly gains: at
+// 3.36 * 10^7 BF16-SR 77.0 -> 75.4, BF16-nearest 79.3 -> 72.4, FP32 115.2 -> 113.7,
+// with FP32 gradients 86.6 -> 83.9; the most it lost was 1.6% (FP32, 4.5 * 10^7
+// elements in twelve tensors, 156.0 -> 158.5).
+constexpr uint64_t kSequenceMinElements = 1ull << 25;
+constexpr uint64_t kSequenceMinElementsUncapped = 5ull << 21;
+
+SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params,
+                                        uint32_t minifloat_sr, uint32_t bytes_per_element) {
+  const bool uncapped = sequence_cap(minifloat_sr, block, lanes, bytes_per_element) == 0;
+  return bf16_params && static_cast<uint64_t>(tiles) * block * lanes >=
+                            (uncapped ? kSequenceMinElementsUncapped : kSequenceMinElements);
 }
 
 // The environment can replace the rule: SR_STATES_RESIDENT_CAP=k caps every

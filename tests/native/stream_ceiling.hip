@@ -277,11 +277,12 @@ extern "C" int sr_stream_ceiling_p(uint64_t n, int p_bytes, int g_bytes, int m_b
   add(0, 0);
   add(0, rule);
   add(0, rule / 2);
-  if (v_bytes && sr::use_sequence(tiles, kBlock, kLanes, p_bytes == 2, per_element)) {
-    // The formats of the states are open: none, one or two may round to FP16
-    // or FP8 stochastically.
+  // The formats of the states are open: none, one or two may round to FP16 or
+  // FP8 stochastically.
+  for (uint32_t moments : {2u, 1u, 0u}) {
+    if (!v_bytes || !sr::use_sequence(tiles, kBlock, kLanes, p_bytes == 2, moments, per_element)) continue;
     add(1, 0);
-    for (uint32_t moments : {2u, 1u, 0u}) add(1, sr::sequence_cap(moments, kBlock, kLanes, per_element));
+    add(1, sr::sequence_cap(moments, kBlock, kLanes, per_element));
     add(1, sr::workgroups_in(sr::sequence_in_flight(0) / 2, kBlock, kLanes, per_element));
   }
   constexpr int kCount = sizeof(kCeilingGaps) / sizeof(kCeilingGaps[0]);

@@ -1,8 +1,8 @@
 """Launches on both sides of the tile-order rule against the C oracle, byte for byte.
 
-AdamW launches with BF16 parameters take their tiles in sequence, with a cap
-on the resident workgroups, from 5 * 2^21 elements on (up to 12 bytes per
-element) or from 2^25 on (more); one tile fewer, in the chunked order.  The
+AdamW launches with BF16 parameters take their tiles in sequence from 5 * 2^21
+elements on, or from 2^25 on where their formats have a cap on the resident
+workgroups there; one tile fewer, in the chunked order.  The
 rule counts whole tiles, so the sizes are chosen by tiles for each workgroup
 size.  The group spreads them over three tensors, each with a partial last
 tile and a remainder; the gradients start off 16-byte alignment.
