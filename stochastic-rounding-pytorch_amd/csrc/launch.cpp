@@ -15,7 +15,7 @@
 //
 // cast_new(x, dtype_code, rule, seed, offset, threads, stream) -> tensor, int or None
 //   cast() into a new contiguous tensor of x's shape and device, allocated
-//   here as torch.empty_like allocates it: about 1.5 us less per call than
+//   here by the call that torch.empty_like makes: about 1.5 us less per call than
 //   allocating in Python.  Returns the tensor, or the entry's status where
 //   that is not 0.  None, with nothing allocated, for an x that is not
 //   exactly a torch.Tensor or Parameter, or under a __torch_function__ mode:
@@ -223,7 +223,9 @@ PyObject* cast_new(PyObject*, PyObject* args) {
   at::Tensor out;
   {
     const pybind11::gil_scoped_release no_gil;
-    out = at::empty_like(x, x.options().dtype(scalar_type(code)), at::MemoryFormat::Contiguous);
+    // The options torch.empty_like(x, dtype=, memory_format=) passes on.
+    out = at::empty_like(x, at::TensorOptions().dtype(scalar_type(code)).pinned_memory(false),
+                         at::MemoryFormat::Contiguous);
   }
   const int64_t n = x.numel();
   if (n == 0) return THPVariable_Wrap(std::move(out));

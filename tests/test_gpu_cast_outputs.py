@@ -5,6 +5,7 @@ from __future__ import annotations
 import pytest
 import torch
 from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from oracle import c_oracle
 
@@ -63,3 +64,23 @@ def test_a_cast_without_room_raises_the_allocator_error(cuda):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert sr_states.cast(x, dtype=torch.bfloat16).count_nonzero() == 0
+
+
+def test_a_dispatch_mode_sees_the_allocation_of_empty_like(cuda):
+    import sr_states
+
+    class Mode(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.calls = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.calls.append((func, dict(kwargs or {})))
+            return func(*args, **(kwargs or {}))
+
+    x = torch.randn(33, 7, device=cuda)
+    with Mode() as expected:
+        torch.empty_like(x, dtype=torch.float16, memory_format=torch.contiguous_format)
+    with Mode() as seen:
+        sr_states.cast(x, dtype=torch.float16, seed=5)
+    assert seen.calls == expected.calls
