@@ -17,15 +17,18 @@
  *     the memory alive until the stream has consumed it.
  *   - Counters are 32-bit: every seed/offset/step word is taken modulo 2^32,
  *     exactly as the reference masks them (sr_states/_hash.py:5-50).
- *   - Large optimizer launches (2^16 tiles or more with FP32 parameters,
- *     5 * 2^21 elements or more with BF16 parameters) reserve dynamic LDS
- *     that their kernels never touch, to keep a measured budget of tiles in
- *     flight per CU, 72 to 104 KiB (none where that allows more than 14
- *     workgroups).  Kernels of other streams running beside such a launch
- *     find that LDS taken on the CUs it occupies.  The environment variable
- *     SR_STATES_RESIDENT_CAP=k (0-16, read once per process) replaces that
- *     rule for every such launch: at most k workgroups per CU, none reserved
- *     for k = 0.  Results do not depend on either.
+ *   - Large optimizer launches (with FP32 parameters 2^16 tiles or more;
+ *     AdamW with BF16 parameters 2^25 elements or more, counted in whole
+ *     tiles) reserve dynamic LDS that their kernels never touch, to keep a
+ *     measured budget of tiles in flight per CU, 72 to 104 KiB; none where
+ *     the formats want more workgroups than that.  Kernels of other streams
+ *     running beside such a launch find that LDS taken on the CUs it
+ *     occupies.  The environment variable SR_STATES_RESIDENT_CAP=k (0-16,
+ *     read once per process) replaces that rule for every optimizer launch
+ *     of 2^16 tiles or more, and for every AdamW launch with BF16 parameters
+ *     that takes its tiles in sequence (5 * 2^21 elements or more where the
+ *     rule has no cap, 2^25 where it has one): at most k workgroups per CU,
+ *     none reserved for k = 0.  Results do not depend on either.
  */
 #ifndef SR_STATES_HIP_H
 #define SR_STATES_HIP_H

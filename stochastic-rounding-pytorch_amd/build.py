@@ -6,7 +6,7 @@ parallel; the shared library is linked in place next to the Python package,
 so it travels with the source tree.  Two CPython extensions over torch's
 tensor type are built alongside it: the host-side group walk
 (csrc/group_walk.cpp -> sr_states/_group_walk<EXT_SUFFIX>) and the native
-entries of the single-tensor launches (csrc/launch.cpp ->
+entries of the launches (csrc/launch.cpp ->
 sr_states/_launch<EXT_SUFFIX>).
 """
 

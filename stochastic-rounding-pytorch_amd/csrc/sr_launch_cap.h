@@ -2,8 +2,8 @@
 //
 // Host code over the HIP runtime, shared by the library's launches and the
 // bandwidth-ceiling helper so that both apply the same launch policy.  How
-// many workgroups to leave resident is sr::resident_cap (sr_tile_order.h);
-// this header turns a cap into the LDS reservation that enforces it.
+// many workgroups to leave resident is sr::resident_cap or sr::sequence_cap
+// (sr_tile_order.h); this header turns a cap into the LDS reservation that enforces it.
 #pragma once
 
 #include <hip/hip_runtime.h>

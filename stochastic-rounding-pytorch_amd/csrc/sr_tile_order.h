@@ -212,7 +212,8 @@ SR_HOST_DEVICE inline uint32_t sequence_cap(uint32_t minifloat_sr, uint32_t bloc
 // arithmetic wants every workgroup: 5 * 2^21.  Two machines, chunked -> in
 // sequence, us, one tensor: E4M3-SR + BF16-SR 23.4 -> 23.2 at 1.05 * 10^7 elements
 // and 41.9 -> 41.0 at 2 * 10^7, E4M3-nearest 19.5 -> 19.2 and 34.2 -> 33.1, two
-// FP16-SR 27.0 -> 27.0 and 48.9 -> 47.5 (72.9 -> 69.7 at 3 * 10^7).
+// FP16-SR 27.0 -> 27.0 and 48.9 -> 47.5 (72.9 -> 69.7 at 3 * 10^7); the most one
+// lost was 2.2% (two FP16-SR, 1.68 * 10^7 in one tensor, 40.9 -> 41.9).
 // Launches with a cap: 2^25.  Below, it depends on the size, by how full the
 // last round of chunks is: BF16-SR 25.8 -> 26.1 at 1.05 * 10^7, 31.6 -> 31.2 at
 // 1.3 * 10^7, 55.6 -> 57.4 at 2.5 * 10^7, 66.9 -> 66.6 at 3 * 10^7; FP32 37.9 ->
