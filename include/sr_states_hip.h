@@ -18,17 +18,19 @@
  *   - Counters are 32-bit: every seed/offset/step word is taken modulo 2^32,
  *     exactly as the reference masks them (sr_states/_hash.py:5-50).
  *   - Large optimizer launches (with FP32 parameters 2^16 tiles or more;
- *     AdamW with BF16 parameters 2^25 elements or more, counted in whole
+ *     AdamW with BF16 parameters 13 * 2^21 elements or more, counted in whole
  *     tiles) reserve dynamic LDS that their kernels never touch, to keep a
  *     measured budget of tiles in flight per CU, 72 to 104 KiB; none where
  *     the formats want more workgroups than that.  Kernels of other streams
  *     running beside such a launch find that LDS taken on the CUs it
  *     occupies.  The environment variable SR_STATES_RESIDENT_CAP=k (0-16,
  *     read once per process) replaces that rule for every optimizer launch
- *     of 2^16 tiles or more, and for every AdamW launch with BF16 parameters
- *     that takes its tiles in sequence (5 * 2^21 elements or more where the
- *     rule has no cap, 2^25 where it has one): at most k workgroups per CU,
- *     none reserved for k = 0.  Results do not depend on either.
+ *     of 2^16 tiles or more, and for the smaller ones with BF16 parameters
+ *     that take their tiles in sequence (AdamW from 5 * 2^21 elements where
+ *     the rule has no cap, from 13 * 2^21 where it has one; SGDM with BF16
+ *     gradients and FP16 or FP8 stochastic momentum from 2^24): at most k
+ *     workgroups per CU, none reserved for k = 0.  Results do not depend on
+ *     either.
  */
 #ifndef SR_STATES_HIP_H
 #define SR_STATES_HIP_H

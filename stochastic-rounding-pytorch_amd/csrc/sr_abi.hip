@@ -141,8 +141,15 @@ int launch_adamw(sr::AdamWArgs& a, int pi, int gi, int me, int ve, int block, vo
 int launch_sgdm(sr::SgdmArgs& a, int pi, int gi, int ue, int block, void* stream) {
   const uint32_t bytes = 2 * sr::enc_bytes(param_enc(pi)) + sr::enc_bytes(param_enc(gi)) + 2 * sr::enc_bytes(ue);
   const int lanes = sr::lane_elements(param_enc(pi), param_enc(gi), ue, ue);
-  return launch(tables().sgdm[pi][gi][ue], block, a.total_tiles, &a, stream, false,
-                chunked_cap(a.total_tiles, block, lanes, bytes, pi == 0, sr::sgdm_in_flight(ue == sr::ENC_F16_SR)));
+  a.in_sequence = sr::use_sequence_sgdm(a.total_tiles, static_cast<uint32_t>(block), static_cast<uint32_t>(lanes),
+                                        pi == 1, gi == 1, minifloat_sr(ue));
+  uint32_t cap;
+  if (a.in_sequence) {
+    cap = cap_override() >= 0 ? static_cast<uint32_t>(cap_override()) : 0u;
+  } else {
+    cap = chunked_cap(a.total_tiles, block, lanes, bytes, pi == 0, sr::sgdm_in_flight(ue == sr::ENC_F16_SR));
+  }
+  return launch(tables().sgdm[pi][gi][ue], block, a.total_tiles, &a, stream, a.in_sequence, cap);
 }
 
 // Tiles of block * lanes elements covering n elements, or fail if they do

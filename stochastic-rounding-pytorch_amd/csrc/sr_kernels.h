@@ -16,8 +16,8 @@
 // BF16 with E5M2-SR m, 13 M 38.8 -> 32.5.  The partial last tile of a row
 // takes whole groups too, and its last lanes the 1-3 elements after them.
 //
-// Tile order (sr_tile_order.h).  Large AdamW launches with BF16 parameters
-// take their tiles in sequence, so that what is in flight on the
+// Tile order (sr_tile_order.h).  Large AdamW launches with BF16 parameters, and
+// some of momentum SGD, take their tiles in sequence, so that what is in flight on the
 // whole chip is one window per stream; all others deal chunks of up to 512
 // consecutive tiles to the XCDs in turn.  Either order with one tile per
 // workgroup beat persistent grid-stride loops.
@@ -68,6 +68,7 @@ struct SgdmArgs {
   SgdmScalars s;
   uint32_t total_tiles;
   uint32_t key_prefix;  // update_key_prefix(seed, rng_step), computed by the host
+  uint32_t in_sequence;  // workgroup b takes tile b; else the chunked order
 };
 
 struct CastArgs {
@@ -325,7 +326,7 @@ __device__ __forceinline__ void sgdm_scalar(char* p, const char* g, char* u, int
 template <int PE, int GE, int UE>
 __global__ __launch_bounds__(kMaxBlock) void sgdm_kernel(const SgdmArgs a) {
   constexpr int E = lane_elements(PE, GE, UE, UE);
-  const uint32_t t = logical_tile(a.total_tiles);
+  const uint32_t t = logical_tile(a.total_tiles, a.in_sequence);
   if (t >= a.total_tiles) return;
   const sr_row r = row_record(a, tile_row_index(a, t));
   char* p = reinterpret_cast<char*>(r.ptr[0]);

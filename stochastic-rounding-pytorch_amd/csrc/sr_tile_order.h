@@ -5,9 +5,10 @@
 // rules for how many workgroups of a large optimizer launch stay resident
 // per CU, with each order's own budgets (at the end).
 //
-// Two orders.  Large AdamW launches with BF16 parameters take their tiles
-// in sequence, workgroup b tile b (use_sequence below); every other launch
-// takes the chunked order that follows.
+// Two orders.  Large AdamW launches with BF16 parameters, and some of momentum
+// SGD, take their tiles in sequence, workgroup b tile b (use_sequence and
+// use_sequence_sgdm below); every other launch takes the chunked order that
+// follows.
 //
 // Chunked order.  The dispatcher hands workgroup b to XCD (b mod 8).  Tiles are dealt to the
 // XCDs in chunks of 2^s consecutive tiles: XCD x takes chunks x, x + 8,
@@ -93,15 +94,9 @@ SR_HOST_DEVICE inline LaunchShape launch_shape(uint32_t tiles, uint32_t block,
 // 6.58, FP32 6.14 -> 6.47 and 6.10 -> 6.39, E4M3-nearest 6.35 -> 6.56 and 6.35
 // -> 6.44.
 //
-// Momentum SGD stays chunked.  With BF16 parameters and gradients, 50 tensors,
-// chunked -> in sequence, us: E4M3-SR momentum 167.9 -> 164.5 at 1.34 * 10^8
-// elements but 561 -> 599 at 4.5 * 10^8, 754 -> 793 at 6 * 10^8 and 1956 -> 2036
-// at 1.55 * 10^9 (E5M2-SR and one tensor alike); FP16-SR 203.1 -> 198.7, 685 ->
-// 695, 914 -> 928 and 2378 -> 2384; FP32 286.5 -> 286.6, 986 -> 985, 1313 -> 1304
-// and 3410 -> 3365; BF16 level.  So do FP32 parameters: over separate allocations
-// the sequence lost 1.8% on GPT-2's shapes with BF16 gradients and 2.3% on 1.55 *
-// 10^9 elements with E4M3-SR + BF16-SR moments, though over flat buffers it
-// gained as much.
+// FP32 parameters stay chunked: over separate allocations the sequence lost 1.8%
+// on GPT-2's shapes with BF16 gradients and 2.3% on 1.55 * 10^9 elements with
+// E4M3-SR + BF16-SR moments, though over flat buffers it gained as much.
 
 // Grid of a launch in sequence: `tiles` workgroups, in rows where one
 // dimension cannot hold them (launch_shape); workgroups past the last tile
@@ -214,15 +209,15 @@ SR_HOST_DEVICE inline uint32_t sequence_cap(uint32_t minifloat_sr, uint32_t bloc
 // and 41.9 -> 41.0 at 2 * 10^7, E4M3-nearest 19.5 -> 19.2 and 34.2 -> 33.1, two
 // FP16-SR 27.0 -> 27.0 and 48.9 -> 47.5 (72.9 -> 69.7 at 3 * 10^7); the most one
 // lost was 2.2% (two FP16-SR, 1.68 * 10^7 in one tensor, 40.9 -> 41.9).
-// Launches with a cap: 2^25.  Below, it depends on the size, by how full the
-// last round of chunks is: BF16-SR 25.8 -> 26.1 at 1.05 * 10^7, 31.6 -> 31.2 at
-// 1.3 * 10^7, 55.6 -> 57.4 at 2.5 * 10^7, 66.9 -> 66.6 at 3 * 10^7; FP32 37.9 ->
-// 39.0, 46.7 -> 46.9, 86.4 -> 86.6, 104.4 -> 102.1; with FP32 gradients 28.5 ->
-// 29.3, 35.1 -> 35.3, 63.6 -> 63.6, 75.8 -> 75.5.  From there it mostly gains: at
-// 3.36 * 10^7 BF16-SR 77.0 -> 75.4, BF16-nearest 79.3 -> 72.4, FP32 115.2 -> 113.7,
-// with FP32 gradients 86.6 -> 83.9; the most it lost was 1.6% (FP32, 4.5 * 10^7
-// elements in twelve tensors, 156.0 -> 158.5).
-constexpr uint64_t kSequenceMinElements = 1ull << 25;
+// Launches with a cap: 13 * 2^21 (27 * 10^6).  Below, it depends on the size, by
+// how full the last round of chunks is: BF16-SR 25.8 -> 26.1 at 1.05 * 10^7, 31.6
+// -> 31.2 at 1.3 * 10^7, 55.6 -> 57.4 at 2.5 * 10^7; FP32 37.9 -> 39.0, 46.7 -> 46.9,
+// 86.4 -> 86.6; with FP32 gradients 28.5 -> 29.3, 35.1 -> 35.3, 63.6 -> 63.6.  From
+// there it mostly gains: at 3 * 10^7 BF16-SR 67.9 -> 66.7, BF16-nearest 67.6 ->
+// 66.1, FP32 104.4 -> 102.1, with FP32 gradients 75.8 -> 75.5; at 3.36 * 10^7 77.0
+// -> 75.4, 79.3 -> 72.4, 115.2 -> 113.7 and 86.6 -> 83.9; the most it lost was 1.6%
+// (FP32, 4.5 * 10^7 elements in twelve tensors, 156.0 -> 158.5).
+constexpr uint64_t kSequenceMinElements = 13ull << 21;
 constexpr uint64_t kSequenceMinElementsUncapped = 5ull << 21;
 
 SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params,
@@ -230,6 +225,24 @@ SR_HOST_DEVICE inline bool use_sequence(uint32_t tiles, uint32_t block, uint32_t
   const bool uncapped = sequence_cap(minifloat_sr, block, lanes, bytes_per_element) == 0;
   return bf16_params && static_cast<uint64_t>(tiles) * block * lanes >=
                             (uncapped ? kSequenceMinElementsUncapped : kSequenceMinElements);
+}
+
+// Whether a momentum-SGD launch takes its tiles in sequence, then without a cap:
+// with momentum that rounds stochastically to FP16 or FP8 and BF16 gradients,
+// from 2^24 to 2^28 elements.  Gain in rate on seven machines, one tensor to fifty:
+// E4M3-SR +0.1 to +1.6% at 1.68 * 10^7, +2.1 to +5.4% at 6.7 * 10^7, +0.7 to +2.3% at
+// 2.7 * 10^8, but -2.4 to -5.2% at 4 * 10^8 and -3 to -6.5% at 6 * 10^8 (754 -> 793
+// us); E5M2-SR alike; FP16-SR +0.4 to +1.5%, +1.1 to +10.8%, +0.9 to +2.1%, then
+// -2.4 to +1.2% and -1.5 to -0.3%.  No others: with FP32 gradients -1.8 to +1.6% in
+// that range, FP32 momentum -2.5 to +1.8%, BF16 momentum level.
+constexpr uint64_t kSequenceSgdmMinElements = 1ull << 24;
+constexpr uint64_t kSequenceSgdmMaxElements = 1ull << 28;
+
+SR_HOST_DEVICE inline bool use_sequence_sgdm(uint32_t tiles, uint32_t block, uint32_t lanes, bool bf16_params,
+                                             bool bf16_gradient, bool minifloat_sr) {
+  const uint64_t elements = static_cast<uint64_t>(tiles) * block * lanes;
+  return bf16_params && bf16_gradient && minifloat_sr && elements >= kSequenceSgdmMinElements &&
+         elements <= kSequenceSgdmMaxElements;
 }
 
 // The environment can replace the rule: SR_STATES_RESIDENT_CAP=k caps every

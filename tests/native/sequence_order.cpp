@@ -29,9 +29,9 @@ int main() {
   }
   // The least elements, each side of the edge: moments that round
   // stochastically to FP16 or FP8, bytes per element, edge.
-  const uint32_t edges[][3] = {{0, 10, 5u << 21}, {0, 12, 5u << 21}, {0, 14, 1u << 25}, {0, 22, 1u << 25},
-                               {1, 12, 5u << 21}, {1, 14, 5u << 21}, {1, 16, 1u << 25}, {2, 14, 5u << 21},
-                               {2, 16, 1u << 25}};
+  const uint32_t edges[][3] = {{0, 10, 5u << 21}, {0, 12, 5u << 21}, {0, 14, 13u << 21}, {0, 22, 13u << 21},
+                               {1, 12, 5u << 21}, {1, 14, 5u << 21}, {1, 16, 13u << 21}, {2, 14, 5u << 21},
+                               {2, 16, 13u << 21}};
   for (uint32_t block : {128u, 256u, 512u, 1024u}) {
     for (const auto& e : edges) {
       const uint32_t edge = e[2] / (block * 4);
@@ -41,6 +41,20 @@ int main() {
         std::printf("block %u, %u moments, %u bytes: the rule's edge moved\n", block, e[0], e[1]);
         ++failures;
       }
+    }
+  }
+  // Momentum SGD: both ends, and the operands.
+  for (uint32_t block : {128u, 256u, 512u, 1024u}) {
+    const uint32_t first = (1u << 24) / (block * 4), last = (1u << 28) / (block * 4);
+    if (!sr::use_sequence_sgdm(first, block, 4, true, true, true) ||
+        sr::use_sequence_sgdm(first - 1, block, 4, true, true, true) ||
+        !sr::use_sequence_sgdm(last, block, 4, true, true, true) ||
+        sr::use_sequence_sgdm(last + 1, block, 4, true, true, true) ||
+        sr::use_sequence_sgdm(first, block, 4, false, true, true) ||
+        sr::use_sequence_sgdm(first, block, 4, true, false, true) ||
+        sr::use_sequence_sgdm(first, block, 4, true, true, false)) {
+      std::printf("block %u: momentum SGD's range moved\n", block);
+      ++failures;
     }
   }
   for (uint32_t bytes = 6; bytes <= 28; ++bytes) {
